@@ -137,6 +137,14 @@ struct PrefillCfg {
     static constexpr int BUF =
         SPV ? KSPLIT * IMG : (STEP_KEYS * KS + STEP_KEYS * HD + 255) / 256 * 256;
     static constexpr int PS_FLOATS = IMG;  // floats per pre-split record
+    // Half images (IEEE-half and E4M3 caches): the lo halves of such rows are all zero, so the
+    // image is the split image without them (hk_chunk, hv_chunk, exponents at float HEXPO), and
+    // each product takes two matrix instructions instead of three: a third of the matrix work
+    // and half of the LDS reads and record bytes were spent on zeros. The same bits; Mistral
+    // 256 rows over 8448 E4M3 keys, the whole call: 122.4 -> 97.6 us, a 1000-row Qwen layer
+    // prompt over a half cache 135.6 -> 129.8.
+    static constexpr int HEXPO = 4 * (KC + 4 * HD);
+    static constexpr int HIMG = SPV ? (HEXPO + 64 + 255) / 256 * 256 : 0;
     // f16 mode (hi halves only): a buffer holds KSPLIT tile images of FIMG floats, each a
     // K part and a V^T part of 16-byte chunks (8 halves) laid out chunk-major: K chunk c
     // (dims 8c .. 8c + 7) of key r at chunk c * 32 + r, V^T chunk c (keys 8c .. 8c + 7 in
@@ -157,9 +165,20 @@ struct PrefillCfg {
     static constexpr size_t LDS_BYTES = (size_t)LDS_FLOATS * sizeof(float);
 };
 
-// Buffer size (floats) of the mode's LDS layout (FAST: tile images of hi halves).
-template <class C, bool FAST>
-constexpr int bufsize() { return FAST ? C::FBUF : C::BUF; }
+// LDS layouts of a tile: split images, the f16 mode's images (FAST), or half images (caches of
+// EB = 2 or 1 bytes an element).
+enum Layout { kSplitImg, kFastImg, kHalfImg };
+template <int HD>
+constexpr Layout layout_of(bool fast, int eb) {
+    return fast ? kFastImg : (eb != 4 && HD >= 32) ? kHalfImg : kSplitImg;
+}
+// Image and buffer sizes of a layout (floats).
+template <class C, Layout L>
+constexpr int imgsize() { return L == kFastImg ? C::FIMG : L == kHalfImg ? C::HIMG : C::IMG; }
+template <class C, Layout L>
+constexpr int bufsize() {
+    return L == kFastImg ? C::FBUF : L == kHalfImg ? C::STEP_KEYS / kTile * C::HIMG : C::BUF;
+}
 
 // f16-mode tile images: the 16-byte chunk index of chunk c of K row r (key r, dims 8c ..
 // 8c + 7), and of chunk c of V^T row p (keys 8c .. 8c + 7).
@@ -174,9 +193,11 @@ template <class C>
 __device__ __forceinline__ int sv_chunk(int p, int c, int lo) {
     return 2 * C::KC + lo * 4 * C::HD_ + c * C::HD_ + p;
 }
-// Image size of the mode (floats).
-template <class C, bool FAST>
-constexpr int imgsize() { return FAST ? C::FIMG : C::IMG; }
+// Half images.
+template <class C>
+__device__ __forceinline__ int hk_chunk(int r, int c) { return c * C::KCS + r; }
+template <class C>
+__device__ __forceinline__ int hv_chunk(int p, int c) { return C::KC + c * C::HD_ + p; }
 
 // Fetch the K and V rows [kb, kb + STEP_KEYS) of KV head kvh into registers; rows past
 // T read as zero. Every element is assigned on every call (clamped addresses, selected
@@ -272,13 +293,18 @@ __device__ __forceinline__ void split_f16(f32x4 x, int e, f16x4 &hi, f16x4 &lo) 
 // arrays) and written as the f16 mode's tile images (fk_chunk, fv_chunk).
 // V16 (with FAST false): K split as above, V rows rounded to f16 as they are, as FAST does
 // (the scores-accurate mode; its V^T lo halves and V exponents are not written).
-template <class C, bool FAST = false, bool V16 = false>
+// HALF: rows of an IEEE-half or E4M3 cache, written as half images. A row scaled into [2^14,
+// 2^15) is exact in f16 but for bits below 2^-24, whose remainder rounds to zero in the lo half
+// too, so the lo half is zero (NaN beside an infinity, which the hi half then takes).
+template <class C, bool FAST = false, bool V16 = false, bool HALF = false>
 __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk)[C::NLD],
                                                    const f32x4 (&rv)[C::NLD], int buf,
                                                    int tid) {
     constexpr int HD = C::HD_;
-    constexpr int IMGX = imgsize<C, FAST>();
-    float *Kb = smem + buf * bufsize<C, FAST>();
+    constexpr Layout LAY = FAST ? kFastImg : HALF ? kHalfImg : kSplitImg;
+    constexpr int IMGX = imgsize<C, LAY>();
+    constexpr int EXPOX = HALF ? C::HEXPO : C::EXPO;
+    float *Kb = smem + buf * bufsize<C, LAY>();
 #pragma unroll
     for (int r = 0; r < C::NLD; ++r) {
         const int idx = tid + r * C::THREADS;
@@ -302,9 +328,13 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                 const int e = split_exponent(mx);
                 f16x4 hi, lo;
                 split_f16(x, e, hi, lo);
-                *reinterpret_cast<f16x4 *>(imh + 8 * sk_chunk<C>(kr, c4 / 2, 0) + (c4 & 1) * 4) = hi;
-                *reinterpret_cast<f16x4 *>(imh + 8 * sk_chunk<C>(kr, c4 / 2, 1) + (c4 & 1) * 4) = lo;
-                if (c4 == 0) reinterpret_cast<int *>(img + C::EXPO)[kr] = e;
+                if constexpr (HALF) {
+                    *reinterpret_cast<f16x4 *>(imh + 8 * hk_chunk<C>(kr, c4 / 2) + (c4 & 1) * 4) = hi + lo;
+                } else {
+                    *reinterpret_cast<f16x4 *>(imh + 8 * sk_chunk<C>(kr, c4 / 2, 0) + (c4 & 1) * 4) = hi;
+                    *reinterpret_cast<f16x4 *>(imh + 8 * sk_chunk<C>(kr, c4 / 2, 1) + (c4 & 1) * 4) = lo;
+                }
+                if (c4 == 0) reinterpret_cast<int *>(img + EXPOX)[kr] = e;
             }
             const f32x4 y = rv[r];
             int ev = 0;
@@ -317,6 +347,7 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                     fmaxf(fmaxf(fabsf(y.x), fabsf(y.y)), fmaxf(fabsf(y.z), fabsf(y.w)));
                 ev = split_exponent(group_max<HD / 4>(vm4));
                 split_f16(y, ev, vh, vl);
+                if constexpr (HALF) vh += vl;
             }
             // V^T row of dim d is p(d) = (d % NB) * 32 + d / NB (the MFMA reader then walks
             // consecutive rows). Keys are stored permuted within each 16: groups of four in
@@ -334,6 +365,8 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                     const int pr = (d % C::NB) * 32 + d / C::NB;
                     if constexpr (FAST) {
                         vimg[8 * fv_chunk<HD>(pr, jc) + jw] = vh[i];
+                    } else if constexpr (HALF) {
+                        vimg[8 * hv_chunk<C>(pr, jc) + jw] = vh[i];
                     } else {
                         vimg[8 * sv_chunk<C>(pr, jc, 0) + jw] = vh[i];
                         if constexpr (!V16) vimg[8 * sv_chunk<C>(pr, jc, 1) + jw] = vl[i];
@@ -346,7 +379,7 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                 using u32x2 = __attribute__((ext_vector_type(2))) unsigned;
                 const u32x2 ho = __builtin_bit_cast(u32x2, vh), lw = __builtin_bit_cast(u32x2, vl);
                 const u32x2 hp = {lane_xor_u<HD / 4>(ho.x), lane_xor_u<HD / 4>(ho.y)};
-                const u32x2 lp = (FAST || V16) ? lw : u32x2{lane_xor_u<HD / 4>(lw.x), lane_xor_u<HD / 4>(lw.y)};
+                const u32x2 lp = (FAST || V16 || HALF) ? lw : u32x2{lane_xor_u<HD / 4>(lw.x), lane_xor_u<HD / 4>(lw.y)};
                 const f16x4 vh2 = __builtin_bit_cast(f16x4, hp), vl2 = __builtin_bit_cast(f16x4, lp);
                 const bool odd = row & 1;
                 const int g4 = (row >> 2) & 3;
@@ -363,6 +396,8 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                     using h2 = __attribute__((ext_vector_type(2))) _Float16;
                     if constexpr (FAST) {
                         vimg[4 * fv_chunk<HD>(pr, jc) + jw] = __builtin_bit_cast(unsigned, h2{he, ho2});
+                    } else if constexpr (HALF) {
+                        vimg[4 * hv_chunk<C>(pr, jc) + jw] = __builtin_bit_cast(unsigned, h2{he, ho2});
                     } else {
                         vimg[4 * sv_chunk<C>(pr, jc, 0) + jw] = __builtin_bit_cast(unsigned, h2{he, ho2});
                         if constexpr (!V16)
@@ -370,7 +405,7 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
                     }
                 }
             }
-            if (!FAST && !V16 && c4 == 0) reinterpret_cast<int *>(img + C::EXPO)[kTile + kr] = ev;
+            if (!FAST && !V16 && c4 == 0) reinterpret_cast<int *>(img + EXPOX)[kTile + kr] = ev;
         } else if (idx < C::STEP_F4) {
             float *Vb = Kb + C::STEP_KEYS * C::KS;
             *reinterpret_cast<f32x4 *>(Kb + row * C::KS + c4 * 4) = rk[r];
@@ -449,7 +484,8 @@ __global__ __launch_bounds__(PresplitCfg<HD>::THREADS) void preconvert_kernel(
 // tile's record. The prefill then only copies records into LDS: the split is done once
 // per key instead of once per workgroup that reads the key.
 
-// V16: records of the scores-accurate mode (V rows rounded to f16 as they are).
+// V16: records of the scores-accurate mode (V rows rounded to f16 as they are). Caches of
+// EB = 2 or 1 bytes an element get half images.
 template <int HD, int EB, bool NT, bool V16 = false>
 __global__ __launch_bounds__(PresplitCfg<HD>::THREADS) void presplit_kernel(
     const void *__restrict__ k, const void *__restrict__ v, float *__restrict__ ps, int nkeys,
@@ -459,7 +495,9 @@ __global__ __launch_bounds__(PresplitCfg<HD>::THREADS) void presplit_kernel(
     static_assert(C::BUF == PrefillCfg<HD, 4, 1, 1>::BUF &&
                       C::PS_FLOATS == PrefillCfg<HD, 4, 1, 1>::PS_FLOATS,
                   "the records' layout is the 32-key step's");
-    __shared__ float smem[C::BUF];
+    constexpr bool HALF = EB != 4;
+    constexpr int IMGX = HALF ? C::HIMG : C::IMG;
+    __shared__ float smem[IMGX];
     const int t = blockIdx.x;
     const int kvh = blockIdx.y;
     const int tid = threadIdx.x;
@@ -467,10 +505,10 @@ __global__ __launch_bounds__(PresplitCfg<HD>::THREADS) void presplit_kernel(
     // halves and V exponents, are left as they are: nothing reads them.)
     f32x4 rk[C::NLD], rv[C::NLD];
     prefill_load_step<C, EB, NT>(k, v, rk, rv, (tlo + t) * kTile, nkeys, Hkv, kvh, tid, hdr);
-    prefill_store_step<C, false, V16>(smem, rk, rv, 0, tid);
+    prefill_store_step<C, false, V16, HALF>(smem, rk, rv, 0, tid);
     __syncthreads();
-    f32x4 *rec = reinterpret_cast<f32x4 *>(ps + ((size_t)kvh * nt + t) * C::PS_FLOATS);
-    for (int c = tid; c < C::IMG / 4; c += C::THREADS)
+    f32x4 *rec = reinterpret_cast<f32x4 *>(ps + ((size_t)kvh * nt + t) * IMGX);
+    for (int c = tid; c < IMGX / 4; c += C::THREADS)
         rec[c] = reinterpret_cast<const f32x4 *>(smem)[c];
 }
 
@@ -488,9 +526,9 @@ __device__ __forceinline__ void wait_vm_keep() {
 // RANGE: queries start at position qbase and may have a sliding window; without it the
 // kernel is specialised to a prompt from position 0 (no window), whose masks are simpler.
 // EB: bytes per K/V element (4 f32, 2 IEEE half, 1 OCP FP8 E4M3: an f16 or E4M3 KV
-// cache), converted to f32 as they are staged.
+// cache), converted to f32 as they are staged; 2 and 1 use half images.
 // PS: K/V come as pre-split records (ps: ps_nt records per KV head, record 0 = tile
-// ps_tlo) instead of k/v.
+// ps_tlo) instead of k/v; with EB 2 the records are half images, of either narrow cache.
 // FAST (an opt-in mode, f32 K/V without pre-split records): q, K, V and P are rounded to
 // f16 once and each product is one f16 MFMA (instead of three on exact hi/lo splits); the
 // online softmax, its rescaling and the accumulation stay f32.
@@ -506,9 +544,10 @@ constexpr bool direct_out() { return FAST && C::STEP_KEYS == kTile && EB_PREFILL
 // FAST3 over records copies each step's images two steps ahead into three buffers.
 template <class C, bool FAST, bool PS>
 constexpr bool triple_buf() { return PS && direct_out<C, FAST>() && EB_PREFILL_FAST_TB; }
-template <class C, bool FAST, bool PS>
+template <class C, bool FAST, bool PS, int EB>
 constexpr size_t prefill_lds_bytes() {
-    constexpr int buf2 = (triple_buf<C, FAST, PS>() ? 3 : 2) * bufsize<C, FAST>();
+    constexpr int buf2 =
+        (triple_buf<C, FAST, PS>() ? 3 : 2) * bufsize<C, layout_of<C::HD_>(FAST, EB)>();
     constexpr int out = direct_out<C, FAST>() ? 0 : C::OUT;
     constexpr int a = buf2 > C::MERGE ? buf2 : C::MERGE;
     return (size_t)(a > out ? a : out) * sizeof(float);
@@ -518,9 +557,9 @@ constexpr int prefill_min_waves() {
     if (direct_out<PrefillCfg<HD, HPW, WPH, KSPLIT>, FAST>() && PS && HD <= 128) return 3;
     return (HPW * WPH * KSPLIT == 4 && HD <= 128) ? 2 : 1;
 }
-template <int HD, int HPW, int WPH, int KSPLIT, bool FAST, bool PS>
+template <int HD, int HPW, int WPH, int KSPLIT, bool FAST, bool PS, int EB>
 constexpr int prefill_max_waves() {
-    constexpr size_t lds = prefill_lds_bytes<PrefillCfg<HD, HPW, WPH, KSPLIT>, FAST, PS>();
+    constexpr size_t lds = prefill_lds_bytes<PrefillCfg<HD, HPW, WPH, KSPLIT>, FAST, PS, EB>();
     constexpr int wgs = lds > 0 ? (int)(kLdsBytesPerCu / lds) : 8;
     constexpr int w = (wgs < 1 ? 1 : wgs) * HPW * WPH * KSPLIT / 4;
     constexpr int lo = prefill_min_waves<HD, HPW, WPH, KSPLIT, FAST, PS>();
@@ -537,7 +576,7 @@ template <int HD, int HPW, int WPH, int KSPLIT, bool RANGE, int EB, bool PS, boo
 __global__ __attribute__((
     amdgpu_flat_work_group_size(1, HPW * WPH * KSPLIT * 64),
     amdgpu_waves_per_eu(prefill_min_waves<HD, HPW, WPH, KSPLIT, FAST, PS>(),
-                        prefill_max_waves<HD, HPW, WPH, KSPLIT, FAST, PS>()))) void prefill_kernel(
+                        prefill_max_waves<HD, HPW, WPH, KSPLIT, FAST, PS, EB>()))) void prefill_kernel(
     const float *__restrict__ q, const void *__restrict__ k, const void *__restrict__ v,
     const float *__restrict__ ps, int ps_tlo, int ps_nt, float *__restrict__ o, int H,
     int Hkv, int rows, int nkeys, int qbase, int window, float scale_log2, int nqb,
@@ -547,7 +586,10 @@ __global__ __attribute__((
     constexpr int HALF = C::HALF;
     constexpr int NB = C::NB;
     constexpr int KS = C::KS;
-    constexpr int BUFX = bufsize<C, FAST>();  // LDS buffer size of this mode
+    constexpr Layout LAY = layout_of<HD>(FAST, EB);
+    constexpr bool HALF16 = LAY == kHalfImg;   // K and V without lo halves
+    constexpr int BUFX = bufsize<C, LAY>();    // LDS buffer size of this mode
+    constexpr int EXPOX = HALF16 ? C::HEXPO : C::EXPO;
 
     extern __shared__ float smem[];  // [2][BUF]: K rows [STEP_KEYS][KS], V rows [STEP_KEYS][HD]
 
@@ -599,7 +641,7 @@ __global__ __attribute__((
     // out right behind the q fragment's, so that the two latencies overlap.
     f32x4 rk[PS ? 1 : C::NLD], rv[PS ? 1 : C::NLD];
     static_assert(!(PS && FAST) || HD <= 128, "f16-mode records for head_dim <= 128");
-    constexpr int IMGX = imgsize<C, FAST>();
+    constexpr int IMGX = imgsize<C, LAY>();
     const float *recs = PS ? ps + (size_t)kvh * ps_nt * IMGX : nullptr;
     // TB: three buffers, the first two steps' copies issued here (a wave's copy of one step
     // is TBL loads; they complete in issue order).
@@ -727,7 +769,7 @@ __global__ __attribute__((
     else if constexpr (PS)
         wait_vm_all();
     else
-        prefill_store_step<C, FAST, PV1>(smem, rk, rv, 0, tid);
+        prefill_store_step<C, FAST, PV1, HALF16>(smem, rk, rv, 0, tid);
     __syncthreads();
 
     // The next step's K/V: PS records straight into the other buffer (which every wave
@@ -745,7 +787,7 @@ __global__ __attribute__((
         if constexpr (PS)
             wait_vm_all();
         else
-            prefill_store_step<C, FAST, PV1>(smem, rk, rv, b1, tid);
+            prefill_store_step<C, FAST, PV1, HALF16>(smem, rk, rv, b1, tid);
     };
 
     if constexpr (C::SPV) {
@@ -761,7 +803,9 @@ __global__ __attribute__((
             // K chunk 2 k2 + hf of key col: hi (FAST: the only) halves, the lo ones 4 HD
             // chunks on
             const _Float16 *kimg = reinterpret_cast<const _Float16 *>(img) +
-                                   8 * (FAST ? fk_chunk<HD>(col, hf) : sk_chunk<C>(col, hf, 0));
+                                   8 * (FAST     ? fk_chunk<HD>(col, hf)
+                                        : HALF16 ? hk_chunk<C>(col, hf)
+                                                 : sk_chunk<C>(col, hf, 0));
             if constexpr (FAST && NKS <= 8) {
                 // All of the tile's K operands are read before the first product (the
                 // compiler would otherwise wait out each read's latency before its product).
@@ -777,6 +821,14 @@ __global__ __attribute__((
                 for (int k2 = 0; k2 < NKS; ++k2)
                     sacc = mfma16(*reinterpret_cast<const f16x8 *>(kimg + 8 * 2 * kTile * k2),
                                   qh[k2], sacc);
+            } else if constexpr (HALF16) {
+                // Two products per 16-dim step: K has no lo half.
+#pragma unroll
+                for (int k2 = 0; k2 < NKS; ++k2) {
+                    const f16x8 ah = *reinterpret_cast<const f16x8 *>(kimg + 8 * 2 * C::KCS * k2);
+                    sacc = mfma16(ah, qh[k2], sacc);
+                    sacc = mfma16(ah, ql[k2], sacc);
+                }
             } else {
                 // Three products per 16-dim step (hi*hi, hi*lo, lo*hi; lo*lo is below 2^-22).
                 // (both operands read before the products with key splits, the lo operand
@@ -799,7 +851,7 @@ __global__ __attribute__((
             // Scores back from the split's units: 2^(eq + ek), ek the exponent of each of
             // this lane's keys (read four at a time).
             if constexpr (!FAST) {
-                const int *Eb = reinterpret_cast<const int *>(img + C::EXPO);
+                const int *Eb = reinterpret_cast<const int *>(img + EXPOX);
 #pragma unroll
                 for (int s4 = 0; s4 < 4; ++s4) {
                     const int4 e4 = *reinterpret_cast<const int4 *>(Eb + 8 * s4 + 4 * hf);
@@ -884,7 +936,7 @@ __global__ __attribute__((
             } else {
                 // The tile's V exponents ev (V row = 2^ev * v').
                 const int *Ev =
-                    reinterpret_cast<const int *>(smem + b * BUFX + ks * IMGX + C::EXPO) + kTile;
+                    reinterpret_cast<const int *>(smem + b * BUFX + ks * IMGX + EXPOX) + kTile;
                 int ev[16];
 #pragma unroll
                 for (int s4 = 0; s4 < 4; ++s4) {
@@ -951,7 +1003,9 @@ __global__ __attribute__((
             // halves, the lo ones 4 HD chunks on
             const _Float16 *vimg =
                 reinterpret_cast<const _Float16 *>(smem + b * BUFX + ks * IMGX) +
-                8 * (FAST ? fv_chunk<HD>(col, hf) : sv_chunk<C>(col, hf, 0));
+                8 * (FAST     ? fv_chunk<HD>(col, hf)
+                     : HALF16 ? hv_chunk<C>(col, hf)
+                              : sv_chunk<C>(col, hf, 0));
             if constexpr (FAST || PV1) {
                 // One product: the NB V fragments of one 16-key half are read first and the
                 // products go round the NB accumulators (measured 2-4 % faster than one
@@ -965,6 +1019,20 @@ __global__ __attribute__((
                         vh[mb] = *reinterpret_cast<const f16x8 *>(vimg + 8 * (2 * u * HD + 32 * mb));
 #pragma unroll
                     for (int mb = 0; mb < NB; ++mb) oacc[mb] = mfma16(vh[mb], ph[u], oacc[mb]);
+                }
+            } else if constexpr (HALF16) {
+                // Two products (V has no lo half); each accumulator's products in the order of
+                // the three-product form, whose third adds zeros: the same bits.
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    f16x8 vh[NB];
+#pragma unroll
+                    for (int mb = 0; mb < NB; ++mb)
+                        vh[mb] = *reinterpret_cast<const f16x8 *>(vimg + 8 * (2 * u * HD + 32 * mb));
+#pragma unroll
+                    for (int mb = 0; mb < NB; ++mb) oacc[mb] = mfma16(vh[mb], ph[u], oacc[mb]);
+#pragma unroll
+                    for (int mb = 0; mb < NB; ++mb) oacc[mb] = mfma16(vh[mb], pl[u], oacc[mb]);
                 }
             } else {
 #pragma unroll
@@ -1537,7 +1605,7 @@ eb_status launch_prefill_r(hipStream_t st, const float *q, const void *k, const 
         attr_err = hipFuncSetAttribute(
             reinterpret_cast<const void *>(
                 &prefill_kernel<HD, HPW, WPH, KSPLIT, RANGE, EB, PS, FAST, PV1>),
-            hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_lds_bytes<C, FAST, PS>());
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)prefill_lds_bytes<C, FAST, PS, EB>());
     });
     if (attr_err != hipSuccess) return eb::hip_fail(attr_err, "hipFuncSetAttribute(prefill)");
     const int g = H / Hkv;
@@ -1545,7 +1613,7 @@ eb_status launch_prefill_r(hipStream_t st, const float *q, const void *k, const 
     const int nqb = (r.rows + C::QB - 1) / C::QB;
     const dim3 grid((unsigned)(nqb * ngroups), (unsigned)ch.nchmax);
     prefill_kernel<HD, HPW, WPH, KSPLIT, RANGE, EB, PS, FAST, PV1>
-        <<<grid, C::THREADS, prefill_lds_bytes<C, FAST, PS>(), st>>>(
+        <<<grid, C::THREADS, prefill_lds_bytes<C, FAST, PS, EB>(), st>>>(
         q, k, v, ps, presplit_tlo(r), presplit_nt(r), o, H, Hkv, r.rows, r.nkeys, r.qbase,
         r.window, scale_log2, nqb, ngroups, ch.ctiles, part_acc, part_ml, r.hdr);
     eb_status err = eb::check_launch("attn_prefill");
@@ -1597,12 +1665,15 @@ eb_status launch_prefill_t(hipStream_t st, const float *q, const void *k, const 
                     k, v, ps, r.nkeys, Hkv, presplit_tlo(r), nt, r.hdr);
             const eb_status err = eb::check_launch("attn_prefill (pre-split)");
             if (err != EB_OK) return err;
-            // (the records are f16 hi/lo splits whatever the cache's element type)
             if constexpr (PV1) {
                 return launch_prefill_r<HD, HPW, WPH, KSPLIT, false, 4, true, false, true>(
                     st, q, k, v, ps, o, H, Hkv, r, scale_log2, ch, part_acc, part_ml);
             } else {
-                if (plain && r.ce == eb::CacheElem::F32)
+                // (half and E4M3 caches share the half images)
+                if (r.ce != eb::CacheElem::F32)
+                    return launch_prefill_r<HD, HPW, WPH, KSPLIT, true, 2, true>(
+                        st, q, k, v, ps, o, H, Hkv, r, scale_log2, ch, part_acc, part_ml);
+                if (plain)
                     return launch_prefill_r<HD, HPW, WPH, KSPLIT, false, 4, true>(
                         st, q, k, v, ps, o, H, Hkv, r, scale_log2, ch, part_acc, part_ml);
                 return launch_prefill_r<HD, HPW, WPH, KSPLIT, true, 4, true>(
