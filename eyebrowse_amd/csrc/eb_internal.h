@@ -175,10 +175,12 @@ eb_status attn_rows_fused(eb_recorder *rec, const eb_tensor *q, const eb_tensor 
 // linear_f16w: y[i][m, o] = sum_k x[m, k] * w[i][o, k] for nseg (1..kLinearMaxSegs)
 // weight/output pairs sharing x; w IEEE half [out_f[i], in_f]. m <= kLinearGemvRows runs
 // the weight-streaming kernel; more rows run the split-f16 matrix-core GEMM, which needs
-// linear_workspace_floats(m, in_f) floats of workspace (row exponents).
+// linear_workspace_floats(m, in_f) floats of workspace (row exponents), and is faster with
+// linear_split_workspace_floats of them (the split rows too), 16-byte aligned.
 constexpr int kLinearMaxSegs = 3;
 constexpr size_t kLinearGemvRows = 8;
 size_t linear_workspace_floats(size_t m, size_t in_f);
+size_t linear_split_workspace_floats(size_t m, size_t in_f);
 eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_t *const *w,
                                    float *const *y, const size_t *out_f, int nseg, size_t m,
                                    size_t in_f, float *ws, size_t ws_floats);

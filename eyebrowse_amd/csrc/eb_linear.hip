@@ -22,6 +22,10 @@
 //    FP32-MFMA GEMM would be capped at 157 TFLOP/s. A pre-pass writes the row exponents.
 //    Rows whose largest magnitude is not finite keep e = 0 and so give a non-finite
 //    result, as the f32 product would.
+//    With a workspace for the split rows (every recorder call), a pre-pass writes x_hi and
+//    x_lo once and linear_tile_kernel copies both and the weight memory-to-LDS; without one
+//    (raw launches, contractions not a multiple of 64) linear_gemm_kernel splits the rows it
+//    stages in every workgroup.
 // A scalar kernel covers shapes the vector paths do not (in % 8 != 0, unaligned
 // pointers), like the reference's odd-width test (matmul.rs:255-272).
 //
@@ -31,6 +35,7 @@
 #include "eb_internal.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <climits>
 #include <mutex>
@@ -473,21 +478,355 @@ __global__ __launch_bounds__(kThreads, MINB) void linear_gemm_kernel(const float
         }
 }
 
-// CUs of the current device (cached per device ordinal).
-int current_cu_count() {
-    static std::mutex mu;
-    static int cache[64] = {};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    std::lock_guard<std::mutex> lk(mu);
-    if (cache[dev] == 0) {
-        int n = 0;
-        cache[dev] = (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
-                          hipSuccess && n > 0)
-                         ? n
-                         : 256;
+// ---------------------------------------------------------------- many rows, split once -
+// Split pass: row i of x scaled by 2^-e_i (linear_row_scale_kernel's exponent, into ex) and
+// split, x_hi into xs row i and x_lo into xs row M + i. One wave per row; rows of up to NC * 512
+// elements stay in registers between the maximum and the split (NC 0: read twice).
+// Bytes: 4 + 4 per element; 4096 x 4096 takes 19.9 us (6.7 TB/s), 64 x 1024 2.5 us (a launch).
+template <int NC>
+__global__ __launch_bounds__(kThreads) void linear_split_kernel(const float *__restrict__ x,
+                                                                _Float16 *__restrict__ xs,
+                                                                float *__restrict__ ex, int M,
+                                                                int K) {
+    const int lane = threadIdx.x & 63;
+    const int row = blockIdx.x * kWaves + (threadIdx.x >> 6);
+    if (row >= M) return;
+    const float *xr = x + (size_t)row * K;
+    const int k8 = K / 8;
+    struct Oct {
+        f32x4 a, b;
+    };
+    auto load = [&](int c) {
+        const float *p = xr + (size_t)(c < k8 ? c : 0) * 8;  // (clamped: a repeat moves no max)
+        return Oct{*reinterpret_cast<const f32x4 *>(p), *reinterpret_cast<const f32x4 *>(p + 4)};
+    };
+    float mx = 0.0f, bad = 0.0f;
+    auto scan = [&](const Oct &v) {
+        mx = fmaxf(mx, fmaxf(fmaxf(fmaxf(fabsf(v.a.x), fabsf(v.a.y)), fmaxf(fabsf(v.a.z), fabsf(v.a.w))),
+                             fmaxf(fmaxf(fabsf(v.b.x), fabsf(v.b.y)), fmaxf(fabsf(v.b.z), fabsf(v.b.w)))));
+        bad += 0.0f * ((v.a.x + v.a.y) + (v.a.z + v.a.w));
+        bad += 0.0f * ((v.b.x + v.b.y) + (v.b.z + v.b.w));
+    };
+    Oct v[NC > 0 ? NC : 1];
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j) v[j] = load(j * 64 + lane);
+#pragma unroll
+        for (int j = 0; j < NC; ++j) scan(v[j]);
+    } else {
+        for (int c = lane; c < k8; c += 64) scan(load(c));
     }
-    return cache[dev];
+    mx = eb::class_reduce<1, true>(mx);
+    bad = eb::class_reduce<1, false>(bad);
+    int e = 0;
+    if (bad == 0.0f && mx > 0.0f) e = ilogbf(mx) - 14;
+    if (lane == 0) ex[row] = (float)e;
+    _Float16 *hi = xs + (size_t)row * K, *lo = hi + (size_t)M * K;
+    auto store = [&](int c, const Oct &o) {
+        typedef float f32x8 __attribute__((ext_vector_type(8)));
+        const f32x8 q = {ldexpf(o.a.x, -e), ldexpf(o.a.y, -e), ldexpf(o.a.z, -e), ldexpf(o.a.w, -e),
+                         ldexpf(o.b.x, -e), ldexpf(o.b.y, -e), ldexpf(o.b.z, -e), ldexpf(o.b.w, -e)};
+        const f16x8 h = __builtin_convertvector(q, f16x8);
+        *reinterpret_cast<f16x8 *>(hi + (size_t)c * 8) = h;
+        *reinterpret_cast<f16x8 *>(lo + (size_t)c * 8) =
+            __builtin_convertvector(q - __builtin_convertvector(h, f32x8), f16x8);
+    };
+    if constexpr (NC > 0) {
+#pragma unroll
+        for (int j = 0; j < NC; ++j)
+            if (j * 64 + lane < k8) store(j * 64 + lane, v[j]);
+    } else {
+        for (int c = lane; c < k8; c += 64) store(c, load(c));
+    }
+}
+
+// Tile shape: WM x WN waves of TM x TN blocks of 32 x 32, times KW waves that share the 16-deep
+// steps of a stage (wave kw takes steps kw, kw + KW, ...), BK of the contraction per stage,
+// NBUF stages in LDS.
+template <int WM_, int WN_, int TM_, int TN_, int KW_, int BK_, int NBUF_>
+struct TileShape {
+    static constexpr int WM = WM_, WN = WN_, TM = TM_, TN = TN_, KW = KW_, BK = BK_, NBUF = NBUF_;
+    static constexpr int NW = WM * WN * KW, THREADS = NW * 64;
+    static constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
+    static constexpr int ROWB = BK * 2;                  // bytes of an LDS row
+    static constexpr int STAGE = (2 * BM + BN) * ROWB;   // x_hi rows, x_lo rows, w rows
+    static constexpr int NI = STAGE / 1024 / NW;         // 1 KiB copies per wave and stage
+    static constexpr int RED = KW > 1 ? NW * TM * TN * 16 * 256 : 0;  // the waves' partial sums
+    static constexpr int LDS = NBUF * STAGE > RED ? NBUF * STAGE : RED;
+    static_assert(STAGE % (1024 * NW) == 0, "every wave issues NI copies per stage");
+    // Waves per SIMD that the LDS allows (the compiler does not see the dynamic LDS).
+    static constexpr int WGS = 160 * 1024 / (LDS + BM * 4);
+    static constexpr int WAVES = WGS * NW / 4 < 1 ? 1 : WGS * NW / 4 > 8 ? 8 : WGS * NW / 4;
+};
+// Chunk c (16 bytes) of LDS row r lies at chunk c ^ tile_swizzle(r) of the row, so that eight
+// consecutive rows' chunks c, read together as an MFMA operand, meet eight different bank groups.
+// The copies keep whole 64- or 128-byte pieces of a row on consecutive lanes.
+template <int BK>
+__device__ __forceinline__ int tile_swizzle(int r) {
+    return BK == 32 ? (r >> 1) & 3 : r & 7;
+}
+
+template <int N>
+__device__ __forceinline__ void wait_copies() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// y tile = x tile . w tile^T from the split rows xs and exponents ex. Requires K % BK == 0, M * K
+// below 2^30, 16-byte aligned xs and w.
+//
+// The operands go memory-to-LDS (global_load_lds: no registers, no arithmetic), NBUF - 1 stages
+// ahead, one barrier per stage. As inline assembly, which the compiler's wait counting does not
+// see; they complete in issue order, so a stage is there when at most the later stages' copies
+// are outstanding. Past the last stage they repeat it (into buffers that nobody reads).
+// What bounds it: tiles of 128 x 256 and up the matrix cores at the clock that the power limit
+// leaves (1.1-1.2 PFLOP/s of f16 products at 4096 x 4096 x 4096; a library f16 product of 8192^3
+// reaches 1.23 here); smaller ones the bytes that a CU can fetch from L2 (about 50 B/ns), hence
+// tiles that balance 2 BM against BN, and as many of them as there are CUs. Against
+// linear_gemm_kernel, which splits x in every workgroup and has no shape for few rows (us, split
+// pass included, q/k/v then o_proj): Qwen 64 rows 22.5 -> 7.9, 32.2 -> 9.7, 1000 rows 52 -> 28,
+// 37.5 -> 23.5; Mistral 64 rows 59 -> 18, 57 -> 16, 500 rows 88 -> 65, 74 -> 48, 4096 rows
+// 420 -> 375, 280 -> 249.
+//
+// With KW > 1 the waves' partial sums meet in LDS, in the order of kw: a result's bits depend on
+// KW, BK and K only, not on the tile.
+// Workgroups: each XCD gets a contiguous range of tiles, in groups of kGroupM row tiles by all
+// feature tiles, row tile fastest, so that the tiles in flight on an XCD share rows and features.
+constexpr int kGroupM = 4;
+template <class C>
+__global__ __attribute__((amdgpu_flat_work_group_size(C::THREADS, C::THREADS),
+                          amdgpu_waves_per_eu(C::WAVES, C::WAVES))) void
+linear_tile_kernel(const _Float16 *__restrict__ xs, const float *__restrict__ ex, LinearSegs s,
+                   int M, int K) {
+    constexpr int BM = C::BM, BN = C::BN, BK = C::BK, TM = C::TM, TN = C::TN, KW = C::KW;
+    constexpr int ROWB = C::ROWB, CPR = BK / 8;  // 16-byte chunks per LDS row
+    extern __shared__ char tile_lds[];
+    __shared__ int s_ex[BM];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nt = gridDim.x, bid = blockIdx.x;
+    const int full = (nt / kXcds) * kXcds;
+    const int t = bid < full ? (bid % kXcds) * (nt / kXcds) + bid / kXcds : bid;
+    const int ntn = s.first[s.nseg], ntm = nt / ntn;
+    const int g0 = t / (kGroupM * ntn) * kGroupM, r0 = t % (kGroupM * ntn);
+    const int gm = min(kGroupM, ntm - g0);  // row tiles of this group
+    const int nu = r0 / gm;
+    const int sg = seg_of(s, nu);
+    const int N = s.n[sg];
+    const int m0 = __builtin_amdgcn_readfirstlane((g0 + r0 % gm) * BM);
+    const int n0 = __builtin_amdgcn_readfirstlane((nu - s.first[sg]) * BN);
+    const _Float16 *w = s.w[sg];
+    for (int i = tid; i < BM; i += C::THREADS) s_ex[i] = (int)ex[min(m0 + i, M - 1)];
+
+    // Copy i of this wave fills KiB block i * NW + wave of the stage; the lane's byte offset
+    // within xs (or w). Rows past the end repeat the last one; they are not stored.
+    unsigned voff[C::NI];
+#pragma unroll
+    for (int i = 0; i < C::NI; ++i) {
+        const int q = (i * C::NW + wave) * 64 + lane;
+        const int row = q / CPR, c = (q % CPR) ^ tile_swizzle<BK>(row);
+        const int xr = min(m0 + (row < BM ? row : row - BM), M - 1) + (row < BM ? 0 : M);
+        const int wr = min(n0 + row - 2 * BM, N - 1);
+        voff[i] = (unsigned)(row < 2 * BM ? xr : wr) * (unsigned)K * 2u + c * 16u;
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) char *)tile_lds;
+    auto copy_stage = [&](int buf, bool more) {
+#pragma unroll
+        for (int i = 0; i < C::NI; ++i) {
+            const int b = i * C::NW + wave;  // (uniform; 2 BM rows are whole blocks)
+            const void *base = b >= 2 * BM * ROWB / 1024 ? static_cast<const void *>(w)
+                                                         : static_cast<const void *>(xs);
+            const unsigned dst = __builtin_amdgcn_readfirstlane(lds0 + buf * C::STAGE + b * 1024);
+            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                         :
+                         : "s"(dst), "v"(voff[i]), "s"(base)
+                         : "memory", "m0");
+        }
+#pragma unroll
+        for (int i = 0; i < C::NI; ++i) voff[i] += more ? 2 * BK : 0;
+    };
+
+    const int kw = wave / (C::WM * C::WN), slot = wave % (C::WM * C::WN);
+    const int wm = slot / C::WN, wn = slot % C::WN;
+    const int hf = lane >> 5, l32 = lane & 31;
+    floatx16 acc[TM][TN];
+#pragma unroll
+    for (int a = 0; a < TM; ++a)
+#pragma unroll
+        for (int b = 0; b < TN; ++b) acc[a][b] = floatx16{};
+
+    const int nst = K / BK;
+#pragma unroll
+    for (int p = 0; p < C::NBUF - 1; ++p) copy_stage(p, p + 1 < nst);
+    constexpr int STEPS = BK / 16 / KW;
+    unsigned off[STEPS];  // the lane's chunk of row l32 in each of its steps
+#pragma unroll
+    for (int j = 0; j < STEPS; ++j)
+        off[j] = l32 * ROWB + ((((j * KW + kw) * 2 + hf) ^ tile_swizzle<BK>(l32)) * 16);
+    int buf = 0, nb = C::NBUF - 1;
+    for (int st = 0; st < nst; ++st) {
+        wait_copies<(C::NBUF - 2) * C::NI>();
+        __syncthreads();  // stage st is there, and nobody reads buffer nb any more
+        copy_stage(nb, st + C::NBUF < nst);
+        const char *xb = tile_lds + buf * C::STAGE + wm * TM * 32 * ROWB;
+        const char *wb = tile_lds + buf * C::STAGE + (2 * BM + wn * TN * 32) * ROWB;
+#pragma unroll
+        for (int j = 0; j < STEPS; ++j) {
+            f16x8 ah[TM], al[TM], bw[TN];
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+                bw[b] = *reinterpret_cast<const f16x8 *>(wb + off[j] + b * 32 * ROWB);
+#pragma unroll
+            for (int a = 0; a < TM; ++a) {
+                ah[a] = *reinterpret_cast<const f16x8 *>(xb + off[j] + a * 32 * ROWB);
+                al[a] = *reinterpret_cast<const f16x8 *>(xb + off[j] + (BM + a * 32) * ROWB);
+            }
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+#pragma unroll
+                for (int b = 0; b < TN; ++b) acc[a][b] = mfma16(ah[a], bw[b], acc[a][b]);
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+#pragma unroll
+                for (int b = 0; b < TN; ++b) acc[a][b] = mfma16(al[a], bw[b], acc[a][b]);
+        }
+        buf = buf == C::NBUF - 1 ? 0 : buf + 1;
+        nb = nb == C::NBUF - 1 ? 0 : nb + 1;
+    }
+    wait_copies<0>();  // (the repeated last stages)
+
+    // Register r of block (a, b): feature l32 of the block, row 8*(r/4) + 4*hf + r%4.
+    float *y = s.y[sg];
+    auto put = [&](int a, int b, int r, float v) {
+        const int o = n0 + (wn * TN + b) * 32 + l32;
+        const int rt = (wm * TM + a) * 32 + 8 * (r >> 2) + 4 * hf + (r & 3);
+        if (m0 + rt < M && o < N) y[(size_t)(m0 + rt) * N + o] = ldexpf(v, s_ex[rt]);
+    };
+    if constexpr (KW == 1) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) put(a, b, r, acc[a][b][r]);
+    } else {
+        constexpr int NR = TM * TN * 16;  // registers of a wave; wave kw sums NR / KW of them
+        __syncthreads();                  // every wave's copies and reads are done
+        float *red = reinterpret_cast<float *>(tile_lds);
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    red[(wave * NR + (a * TN + b) * 16 + r) * 64 + lane] = acc[a][b][r];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NR / KW; ++i) {
+            const int f = kw * (NR / KW) + i;
+            float v = red[(slot * NR + f) * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < KW; ++k) v += red[((k * C::WM * C::WN + slot) * NR + f) * 64 + lane];
+            put(f / 16 / TN, f / 16 % TN, f % 16, v);
+        }
+    }
+}
+
+template <class C>
+eb_status launch_tile(hipStream_t st, const _Float16 *xs, const float *ex, LinearSegs s,
+                      const size_t *out_f, int nseg, size_t m, size_t in_f) {
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    std::call_once(once, [] {
+        attr_err = hipFuncSetAttribute(reinterpret_cast<const void *>(&linear_tile_kernel<C>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+    });
+    if (attr_err != hipSuccess) return eb::hip_fail(attr_err, "hipFuncSetAttribute(linear)");
+    s.first[0] = 0;
+    for (int i = 0; i < nseg; ++i)
+        s.first[i + 1] = s.first[i] + (int)((out_f[i] + C::BN - 1) / C::BN);
+    const size_t tiles = (m + C::BM - 1) / C::BM * (size_t)s.first[nseg];
+    linear_tile_kernel<C><<<(unsigned)tiles, C::THREADS, C::LDS, st>>>(xs, ex, s, (int)m, (int)in_f);
+    return eb::check_launch("linear_f16w");
+}
+
+// The tile shapes, and the time of one round of tiles (one per CU) as fixed + per_k * K us, fitted
+// to a sweep of 9 to 4096 rows at the Qwen and Mistral widths. tile_cost takes the rounds of the
+// fullest CU, or half way to the average where two workgroups share a CU and overlap.
+struct TileModel {
+    int bm, bn;
+    bool shared;  // two workgroups per CU
+    float fixed, per_k;
+};
+// Up to kTileFewRows rows and whole 128-deep stages: eight waves share each stage's steps, which
+// keeps a CU's copies in flight on the small tiles that few rows need (Qwen o_proj, 256 rows: 11.6
+// us, against 18.9 with the one-sum shapes). Beyond, one chain of sums per output.
+using TileK8a = TileShape<1, 1, 1, 1, 8, 128, 4>;
+using TileK8b = TileShape<1, 1, 1, 2, 8, 128, 4>;
+using TileK8c = TileShape<1, 1, 2, 2, 8, 128, 3>;
+using TileA = TileShape<2, 2, 1, 1, 1, 64, 3>;
+using TileB = TileShape<2, 4, 1, 1, 1, 64, 2>;
+using TileC = TileShape<4, 2, 1, 2, 1, 64, 3>;
+using TileD = TileShape<2, 4, 2, 2, 1, 32, 2>;
+using TileE = TileShape<4, 2, 2, 4, 1, 32, 3>;
+constexpr size_t kTileFewRows = 256;
+constexpr TileModel kTilesK8[] = {{32, 32, false, 1.5f, 2.33e-3f},
+                                  {32, 64, false, 2.2f, 2.9e-3f},
+                                  {64, 64, false, 3.6f, 4.75e-3f}};
+constexpr TileModel kTiles[] = {{64, 64, true, 3.0f, 5.2e-3f},
+                                {64, 128, true, 4.0f, 8.0e-3f},
+                                {128, 128, false, 5.0f, 15.2e-3f},
+                                {128, 256, true, 6.0f, 27.5e-3f},
+                                {256, 256, false, 12.0f, 53.0e-3f}};
+float tile_cost(const TileModel &t, const size_t *out_f, int nseg, size_t m, size_t in_f, float cus) {
+    size_t units = 0;
+    for (int i = 0; i < nseg; ++i) units += (out_f[i] + t.bn - 1) / t.bn;
+    const float avg = (float)((m + t.bm - 1) / t.bm * units) / cus;
+    float rounds = std::ceil(avg);
+    if (t.shared && avg > 1.0f) rounds = 0.5f * (rounds + avg);
+    return rounds * (t.fixed + t.per_k * (float)in_f);
+}
+template <size_t NT>
+int best_tile(const TileModel (&tiles)[NT], const size_t *out_f, int nseg, size_t m, size_t in_f) {
+    const float cus = (float)eb::current_cu_count();
+    int best = 0;
+    float cost = 0.0f;
+    for (int i = 0; i < (int)NT; ++i) {
+        const float c = tile_cost(tiles[i], out_f, nseg, m, in_f, cus);
+        if (i == 0 || c < cost) cost = c, best = i;
+    }
+    return best;
+}
+
+// Floats ahead of the split rows: the row exponents, to whole 256-byte lines.
+size_t tile_ex_floats(size_t m) { return (m + 63) / 64 * 64; }
+
+eb_status launch_tiles(hipStream_t st, const float *x, const LinearSegs &s, const size_t *out_f,
+                       int nseg, size_t m, size_t in_f, float *ws) {
+    float *ex = ws;
+    _Float16 *xs = reinterpret_cast<_Float16 *>(ws + tile_ex_floats(m));
+    const unsigned grid = (unsigned)((m + kWaves - 1) / kWaves);
+    const int M = (int)m, K = (int)in_f;
+    if (K <= 1024) linear_split_kernel<2><<<grid, kThreads, 0, st>>>(x, xs, ex, M, K);
+    else if (K <= 2048) linear_split_kernel<4><<<grid, kThreads, 0, st>>>(x, xs, ex, M, K);
+    else if (K <= 4096) linear_split_kernel<8><<<grid, kThreads, 0, st>>>(x, xs, ex, M, K);
+    else linear_split_kernel<0><<<grid, kThreads, 0, st>>>(x, xs, ex, M, K);
+    const eb_status err = eb::check_launch("linear_f16w (split pass)");
+    if (err != EB_OK) return err;
+    if (m <= kTileFewRows && in_f % 128 == 0) {
+        switch (best_tile(kTilesK8, out_f, nseg, m, in_f)) {
+            case 0: return launch_tile<TileK8a>(st, xs, ex, s, out_f, nseg, m, in_f);
+            case 1: return launch_tile<TileK8b>(st, xs, ex, s, out_f, nseg, m, in_f);
+            default: return launch_tile<TileK8c>(st, xs, ex, s, out_f, nseg, m, in_f);
+        }
+    }
+    switch (best_tile(kTiles, out_f, nseg, m, in_f)) {
+        case 0: return launch_tile<TileA>(st, xs, ex, s, out_f, nseg, m, in_f);
+        case 1: return launch_tile<TileB>(st, xs, ex, s, out_f, nseg, m, in_f);
+        case 2: return launch_tile<TileC>(st, xs, ex, s, out_f, nseg, m, in_f);
+        case 3: return launch_tile<TileD>(st, xs, ex, s, out_f, nseg, m, in_f);
+        default: return launch_tile<TileE>(st, xs, ex, s, out_f, nseg, m, in_f);
+    }
 }
 
 // ksplit 2 expects the outputs zeroed (linear_row_scale_kernel's zero_out).
@@ -526,6 +865,13 @@ namespace eb {
 
 size_t linear_workspace_floats(size_t m, size_t in_f) {
     return (m > kLinearGemvRows && in_f % 8 == 0) ? m : 0;
+}
+
+// (M * K below 2^30: the split rows' byte offsets are 32 bits.)
+size_t linear_split_workspace_floats(size_t m, size_t in_f) {
+    if (m <= kLinearGemvRows || in_f == 0 || in_f % 64 != 0 || m > ((size_t)1 << 30) / in_f - 1)
+        return linear_workspace_floats(m, in_f);
+    return tile_ex_floats(m) + m * in_f;
 }
 
 eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_t *const *w,
@@ -582,6 +928,10 @@ eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_
         return check_launch("linear_f16w");
     }
     if (ws == nullptr || ws_floats < m) return fail(EB_SHAPE_MISMATCH, "linear: workspace too small");
+    const size_t split = linear_split_workspace_floats(m, in_f);
+    if (split > linear_workspace_floats(m, in_f) && ws_floats >= split && aligned16(ws))
+        return launch_tiles(st, x, s, out_f, nseg, m, in_f, ws);
+    // Without a workspace for the split rows.
     // Wide tiles (64 x 128 per wave: 0.5 LDS fragment reads per MFMA instead of 0.75) when
     // they still give every CU two workgroups; otherwise 128 x 128 tiles, whose twice as
     // many workgroups keep more of the chip busy. With at most one 128 x 128 tile per CU

@@ -1016,6 +1016,12 @@ static eb_status device_workspace(eb_device *dev, size_t floats, float **out, Ws
     return EB_OK;
 }
 
+// Whether the device's workspace already holds that many floats.
+static bool workspace_holds(eb_device *dev, size_t floats) {
+    std::lock_guard<std::mutex> lk(dev->ws_mu);
+    return dev->ws_floats >= floats;
+}
+
 // Shared by eb_attn_decode / eb_attn_decode_step: device workspace, then one launch.
 static eb_status device_decode(eb_device *dev, const float *q, const void *kc, const void *vc,
                                void *kc_w, void *vc_w, const float *knew, const float *vnew,
@@ -1092,10 +1098,23 @@ static eb_status device_linear(eb_device *dev, const eb_tensor *a,
         yp[i] = static_cast<float *>(c[i]->ptr);
         yn[i] = eb_tensor_numel(c[i]);
     }
-    const size_t wsn = eb::linear_workspace_floats(m, in_f);
+    // Room for the split rows, or for the row exponents alone where the workspace cannot grow
+    // that far (during a capture, or without the memory).
+    size_t wsn = eb::linear_split_workspace_floats(m, in_f);
     float *ws = nullptr;
     WsLock lk;
-    if (wsn > 0) EB_TRY(device_workspace(dev, wsn, &ws, lk));
+    if (wsn > 0) {
+        const size_t least = eb::linear_workspace_floats(m, in_f);
+        if (dev->capturing.load() && !workspace_holds(dev, wsn)) wsn = least;
+        eb_status st = device_workspace(dev, wsn, &ws, lk);
+        if (st == EB_OUT_OF_MEMORY && wsn > least) {
+            (void)hipGetLastError();  // (reported by no later call)
+            lk.unlock();
+            wsn = least;
+            st = device_workspace(dev, wsn, &ws, lk);
+        }
+        if (st != EB_OK) return st;
+    }
     return linear_checked(dev->stream, static_cast<const float *>(a->ptr), eb_tensor_numel(a),
                           wp, wh, yp, yn, out_f, nseg, m, in_f, ws, wsn);
 }

@@ -1,0 +1,136 @@
+"""linear_f16w on split rows copied memory-to-LDS (linear_tile_kernel): every tile shape at its
+edges against the oracle, the same bits whatever the launch's other outputs, and the path
+without room for the split rows."""
+import numpy as np
+import pytest
+
+import eyebrowse_amd as eb
+import oracle
+from tests._gpu import assert_bitwise, assert_close, note, upload
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return eb.Device.new(0)
+
+
+def _run(dev, x, ws, m, in_f):
+    """One launch for all of ws; the outputs start as NaN, so an element left out shows."""
+    xt = upload(dev, x)
+    wts = [eb.Tensor.from_f16_packed(dev, w.shape, w) for w in ws]
+    cs = [upload(dev, np.full((m, w.shape[0]), np.nan, np.float32)) for w in ws]
+    rec = eb.Recorder(dev)
+    eb.linear_f16w_multi(rec, xt, wts, cs, [w.shape[0] for w in ws], m, in_f)
+    rec.submit()
+    return [c.to_f32().reshape(m, -1) for c in cs]
+
+
+# (rows, contraction, features of each output): which shape runs follows the cost model; the
+# sizes put the rows and features on, below and above its 32 .. 256 edges.
+CASES = [
+    (9, 128, (1,)), (31, 256, (33, 32)), (32, 1024, (4096,)), (33, 128, (31, 65, 64)),   # 32 x 32
+    (65, 4096, (1000, 513)), (96, 1024, (4095,)),                                          # 32 x 64
+    (255, 1024, (4100, 63)), (256, 128, (20000,)),                                         # 64 x 64
+    (9, 64, (40,)), (40, 192, (129,)), (257, 64, (64, 1)), (319, 1024, (1001,)),           # one sum
+    (513, 128, (2049, 100)), (700, 1024, (4095,)), (1025, 2048, (1025,)),
+    (1000, 4096, (4095, 1)), (2049, 64, (4097,)), (2000, 1024, (4096, 250)), (4095, 1024, (4090,)),
+    (300, 8256, (300,)),                                                                   # rows read twice
+]
+
+
+@pytest.mark.parametrize("m,in_f,outs", CASES)
+def test_tiles_match_oracle(dev, m, in_f, outs):
+    note(f"linear tiles m={m} in={in_f} outs={outs}")
+    x = oracle.randn((m, in_f), 1)
+    x[::3] *= np.float32(1e-6)   # rows of their own scale
+    ws = [oracle.randn((o, in_f), 2 + i) * np.float32(in_f ** -0.5) for i, o in enumerate(outs)]
+    got = _run(dev, x, ws, m, in_f)
+    rows = sorted({r for r in (0, 1, 31, 32, 63, 64, 127, 128, 255, 256, m // 2, m - 2, m - 1)
+                   if 0 <= r < m})
+    for g, w in zip(got, ws):
+        assert np.isfinite(g).all()
+        want = oracle.linear_f16w(x[rows], oracle.f16_bits(w), len(rows), in_f, w.shape[0],
+                                  threads=16)
+        scale = np.abs(x[rows]).max(1, keepdims=True)
+        assert_close(g[rows] / scale, want / scale, what=f"{w.shape[0]} features")
+
+
+@pytest.mark.parametrize("m", [40, 256, 257, 700])
+def test_bits_do_not_depend_on_the_launch(dev, m):
+    """An output's sums are the same whether it is launched alone or beside others (other tile
+    shapes)."""
+    note(f"linear tiles alone and together m={m}")
+    in_f, outs = 1024, (2048, 100, 3000)
+    x = oracle.randn((m, in_f), 5)
+    ws = [oracle.randn((o, in_f), 6 + i) * np.float32(0.03) for i, o in enumerate(outs)]
+    together = _run(dev, x, ws, m, in_f)
+    for t, w in zip(together, ws):
+        assert_bitwise(_run(dev, x, [w], m, in_f)[0], t, f"{w.shape[0]} features")
+
+
+def test_extreme_rows(dev):
+    """Row scales from 1e-38 to 1e30, zeros, infinities and NaN, as on the other path."""
+    note("linear tiles extreme rows")
+    m, in_f, out_f = 40, 256, 96
+    x = oracle.randn((m, in_f), 7)
+    for i in range(30):
+        x[i] *= np.float32(10.0 ** (-37 + 2.3 * i))
+    x[30] = 0.0
+    x[31, 5], x[32, 9] = np.inf, np.nan
+    w = oracle.randn((out_f, in_f), 8) * np.float32(0.05)
+    got = _run(dev, x, [w], m, in_f)[0]
+    want = oracle.linear_f16w(x, oracle.f16_bits(w), m, in_f, out_f, threads=16)
+    for i in list(range(30)) + list(range(33, 40)):
+        scale = float(np.max(np.abs(want[i])))
+        assert_close(got[i] / scale, want[i] / scale, what=f"row {i}")
+    assert np.array_equal(got[30], np.zeros(out_f, np.float32))
+    assert not np.isfinite(got[31:33]).any()
+
+
+def test_capture_without_room_for_the_split_rows():
+    """A capture that can use the workspace as it is, but not grow it, still records the product
+    (with the exponents alone); replays give its result."""
+    note("linear tiles capture without room")
+    dev = eb.Device.new(0)
+    m, in_f, out_f = 12, 256, 80
+    xs = oracle.randn((16, 40), 1)
+    rec = eb.Recorder(dev)
+    c0 = eb.Tensor.empty(dev, (16, 8))
+    eb.linear_f16w(rec, upload(dev, xs), eb.Tensor.from_f16_packed(dev, (8, 40), oracle.randn((8, 40), 2)),
+                   c0, 16, 40, 8)   # leaves a workspace of 16 floats
+    rec.submit()
+    x = oracle.randn((m, in_f), 3)
+    w = oracle.randn((out_f, in_f), 4) * np.float32(0.05)
+    xt, wt = upload(dev, x), eb.Tensor.from_f16_packed(dev, w.shape, w)
+    ct = upload(dev, np.full((m, out_f), np.nan, np.float32))
+    dev.begin_capture()
+    rec = eb.Recorder(dev)
+    eb.linear_f16w(rec, xt, wt, ct, m, in_f, out_f)
+    rec.submit()
+    g = dev.end_capture()
+    want = oracle.linear_f16w(x, oracle.f16_bits(w), m, in_f, out_f, threads=16)
+    for _ in range(3):
+        ct.write(np.full((m, out_f), np.nan, np.float32))
+        g.launch()
+        dev.synchronize()
+        assert_close(ct.to_f32().reshape(m, out_f), want, what="replay")
+    g.release()
+
+
+def test_raw_launch_with_room_for_the_split_rows(dev):
+    """A raw launch given m exponents (to whole 64 floats) and the split rows takes the same path
+    as the recorder."""
+    note("linear tiles raw")
+    m, in_f, out_f = 50, 1024, 320
+    x = oracle.randn((m, in_f), 20)
+    w = oracle.randn((out_f, in_f), 21) * np.float32(0.05)
+    xt, wt = upload(dev, x), eb.Tensor.from_f16_packed(dev, w.shape, w)
+    ct = eb.Tensor.empty(dev, (m, out_f))
+    n = 64 + m * in_f
+    ws = upload(dev, np.full(n, np.nan, np.float32))
+    eb.launch_linear_f16w(dev.stream, xt.data_ptr, xt.numel(), wt.data_ptr, 2 * wt.numel(),
+                          ct.data_ptr, ct.numel(), m, in_f, out_f, ws.data_ptr, n)
+    dev.synchronize()
+    assert_bitwise(ct.to_f32(), _run(dev, x, [w], m, in_f)[0], "raw against recorder")
