@@ -551,6 +551,9 @@ struct TileShape {
     static constexpr int ROWB = BK * 2;                  // bytes of an LDS row
     static constexpr int STAGE = (2 * BM + BN) * ROWB;   // x_hi rows, x_lo rows, w rows
     static constexpr int NI = STAGE / 1024 / NW;         // 1 KiB copies per wave and stage
+    // One wave per output: the contraction's halves are summed apart where the registers hold two
+    // sums (see linear_tile_kernel).
+    static constexpr bool HALVES = KW == 1 && TM * TN <= 2;
     static constexpr int RED = KW > 1 ? NW * TM * TN * 16 * 256 : 0;  // the waves' partial sums
     static constexpr int LDS = NBUF * STAGE > RED ? NBUF * STAGE : RED;
     static_assert(STAGE % (1024 * NW) == 0, "every wave issues NI copies per stage");
@@ -572,7 +575,7 @@ __device__ __forceinline__ void wait_copies() {
 }
 
 // y tile = x tile . w tile^T from the split rows xs and exponents ex. Requires K % BK == 0, M * K
-// below 2^30, 16-byte aligned xs and w.
+// below 2^30, N * K below 2^31 (as every launch's weight is), 16-byte aligned xs and w.
 //
 // The operands go memory-to-LDS (global_load_lds: no registers, no arithmetic), NBUF - 1 stages
 // ahead, one barrier per stage. As inline assembly, which the compiler's wait counting does not
@@ -587,8 +590,13 @@ __device__ __forceinline__ void wait_copies() {
 // 37.5 -> 23.5; Mistral 64 rows 59 -> 18, 57 -> 16, 500 rows 88 -> 65, 74 -> 48, 4096 rows
 // 420 -> 375, 280 -> 249.
 //
-// With KW > 1 the waves' partial sums meet in LDS, in the order of kw: a result's bits depend on
-// KW, BK and K only, not on the tile.
+// With KW > 1 the waves' partial sums meet in LDS, in the order of kw. With one wave per output
+// (KW 1) and up to two blocks of accumulators, the first half of the contraction is set aside
+// half way and added at the end: the roundings of a sum are half as many, of half the size
+// (relative error against 64 bits 2.9e-7 in one chain, 2.1e-7 in two at K 1024, 5.8e-7 and
+// 4.1e-7 at 4096). linear_gemm_kernel cuts the contraction at the sizes that these shapes take;
+// the larger shapes keep one chain, as its wide tiles do. A result's bits depend on KW, HALVES,
+// BK and K only, not on the tile.
 // Workgroups: each XCD gets a contiguous range of tiles, in groups of kGroupM row tiles by all
 // feature tiles, row tile fastest, so that the tiles in flight on an XCD share rows and features.
 constexpr int kGroupM = 4;
@@ -664,7 +672,14 @@ linear_tile_kernel(const _Float16 *__restrict__ xs, const float *__restrict__ ex
     for (int j = 0; j < STEPS; ++j)
         off[j] = l32 * ROWB + ((((j * KW + kw) * 2 + hf) ^ tile_swizzle<BK>(l32)) * 16);
     int buf = 0, nb = C::NBUF - 1;
+    floatx16 first[C::HALVES ? TM : 1][C::HALVES ? TN : 1] = {};
     for (int st = 0; st < nst; ++st) {
+        if (C::HALVES && st == nst / 2) {
+#pragma unroll
+            for (int a = 0; a < TM; ++a)
+#pragma unroll
+                for (int b = 0; b < TN; ++b) first[a][b] = acc[a][b], acc[a][b] = floatx16{};
+        }
         wait_copies<(C::NBUF - 2) * C::NI>();
         __syncthreads();  // stage st is there, and nobody reads buffer nb any more
         copy_stage(nb, st + C::NBUF < nst);
@@ -694,6 +709,12 @@ linear_tile_kernel(const _Float16 *__restrict__ xs, const float *__restrict__ ex
         nb = nb == C::NBUF - 1 ? 0 : nb + 1;
     }
     wait_copies<0>();  // (the repeated last stages)
+    if constexpr (C::HALVES) {
+#pragma unroll
+        for (int a = 0; a < TM; ++a)
+#pragma unroll
+            for (int b = 0; b < TN; ++b) acc[a][b] = first[a][b] + acc[a][b];
+    }
 
     // Register r of block (a, b): feature l32 of the block, row 8*(r/4) + 4*hf + r%4.
     float *y = s.y[sg];

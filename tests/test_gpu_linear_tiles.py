@@ -134,3 +134,18 @@ def test_raw_launch_with_room_for_the_split_rows(dev):
                           ct.data_ptr, ct.numel(), m, in_f, out_f, ws.data_ptr, n)
     dev.synchronize()
     assert_bitwise(ct.to_f32(), _run(dev, x, [w], m, in_f)[0], "raw against recorder")
+
+
+@pytest.mark.parametrize("m,in_f,limit", [(300, 1024, 2.5e-7), (1000, 1024, 2.5e-7), (300, 4096, 4.9e-7)])
+def test_sums_are_cut_in_two(dev, m, in_f, limit):
+    """Rows past the few that several waves share: the error against 64 bits is that of two chains
+    of sums, not of one. Each chain's roundings are half as many, of half the size, so one chain
+    is sqrt(2) further off (measured: 2.1e-7 and 2.9e-7 at 1024, 4.1e-7 and 5.8e-7 at 4096, each
+    within 1 % over sizes and inputs); the limit lies half way."""
+    note(f"linear tiles precision m={m} in={in_f}")
+    x = oracle.randn((m, in_f), 30)
+    w = (oracle.randn((1024, in_f), 31) * np.float32(in_f ** -0.5)).astype(np.float16)
+    got = _run(dev, x, [w.astype(np.float32)], m, in_f)[0].astype(np.float64)
+    want = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert err <= limit, err
