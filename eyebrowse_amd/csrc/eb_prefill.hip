@@ -93,6 +93,15 @@ constexpr int kTile = 32;  // keys per tile, queries per wave
 constexpr size_t kLdsBytesPerCu = 160 * 1024;  // gfx950 LDS per CU
 constexpr float kSlack = 8.0f;  // log2 units the reference max may lag a score (SPV)
 constexpr int kUnitSlack = 8;   // bits a P V term may exceed its query's O^T unit (SPV)
+// K and V operands read from LDS ahead of their products, in 16-deep steps (kernels over
+// records, except the f16 mode, which reads all of a tile's K operands first). The compiler
+// waited for each read right after its issue: with one wave per SIMD (head_dim 256) nothing
+// else ran meanwhile. Measured, none -> 2 (us): Gemma-4 prompt of 2000 rows 186.6 -> 177.4,
+// 4096 492 -> 472, 1000 over E4M3 75.3 -> 71.6, Qwen 4096 380 -> 371, Mistral 4096 1093 -> 1086.
+// 1 / 2 ahead for K / V 187.2, 2 / 1 184.5, 2 / 3 178.6, 4 / 4 179.6, 6 / 6 182.5 (Gemma-4,
+// 2000 rows: beyond 2 the registers run out and more of q is copied from AGPRs). The staged
+// kernels' registers are taken by the staging.
+constexpr int kOperandsAhead = 2;
 
 __device__ __forceinline__ floatx16 mfma32(float a, float b, floatx16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
@@ -797,6 +806,24 @@ __global__ __attribute__((
         //  softmax: the online softmax update (m, l, the O^T unit E, the rescale of O^T) and
         //           the P^T operands;
         //  pv:      O^T += V^T P^T from buffer b.
+        constexpr int KA = !FAST && PS ? kOperandsAhead : 0, VA = PV1 ? 0 : KA;
+        constexpr int kSchedAlu = 0x6;  // (vector and scalar arithmetic may move across)
+        f16x8 vh_[VA > 0 ? VA : 1], vl_[VA > 0 ? VA : 1];
+        // V^T fragment f: keys of half f % 2, block f / 2.
+        auto read_v = [&](int b, int f) {
+            const _Float16 *vp = reinterpret_cast<const _Float16 *>(smem + b * BUFX + ks * IMGX) +
+                                 8 * (HALF16 ? hv_chunk<C>(col, hf) : sv_chunk<C>(col, hf, 0)) +
+                                 8 * (2 * (f % 2) * HD + 32 * (f / 2));
+            vh_[f % VA] = *reinterpret_cast<const f16x8 *>(vp);
+            if constexpr (!HALF16) vl_[f % VA] = *reinterpret_cast<const f16x8 *>(vp + 8 * 4 * HD);
+        };
+        auto preread_v = [&](int b) {
+            if constexpr (VA > 0) {
+#pragma unroll
+                for (int f = 0; f < (VA < 2 * NB ? VA : 2 * NB); ++f) read_v(b, f);
+                __builtin_amdgcn_sched_barrier(kSchedAlu);
+            }
+        };
         auto tile_qk = [&](int b, floatx16 &sacc) {
             const float *img = smem + b * BUFX + ks * IMGX;  // tile ks's image
 #pragma unroll
@@ -822,6 +849,30 @@ __global__ __attribute__((
                 for (int k2 = 0; k2 < NKS; ++k2)
                     sacc = mfma16(*reinterpret_cast<const f16x8 *>(kimg + 8 * 2 * kTile * k2),
                                   qh[k2], sacc);
+            } else if constexpr (KA > 0) {
+                // Products per 16-dim step: hi*hi, hi*lo, lo*hi (lo*lo is below 2^-22; half
+                // images have no lo half, so two). The K operands of the next KA steps are read
+                // ahead of them.
+                constexpr int KN = KA < NKS ? KA : NKS;
+                f16x8 ah[KN], al[KN];
+                auto read_k = [&](int k2) {
+                    const _Float16 *kh = kimg + 8 * 2 * C::KCS * k2;
+                    ah[k2 % KN] = *reinterpret_cast<const f16x8 *>(kh);
+                    if constexpr (!HALF16)
+                        al[k2 % KN] = *reinterpret_cast<const f16x8 *>(kh + 8 * C::KC);
+                };
+#pragma unroll
+                for (int k2 = 0; k2 < KN; ++k2) read_k(k2);
+                __builtin_amdgcn_sched_barrier(kSchedAlu);
+#pragma unroll
+                for (int k2 = 0; k2 < NKS; ++k2) {
+                    sacc = mfma16(ah[k2 % KN], qh[k2], sacc);
+                    sacc = mfma16(ah[k2 % KN], ql[k2], sacc);
+                    if constexpr (!HALF16) sacc = mfma16(al[k2 % KN], qh[k2], sacc);
+                    __builtin_amdgcn_sched_barrier(kSchedAlu);
+                    if (k2 + KN < NKS) read_k(k2 + KN);
+                    __builtin_amdgcn_sched_barrier(kSchedAlu);
+                }
             } else if constexpr (HALF16) {
                 // Two products per 16-dim step: K has no lo half.
 #pragma unroll
@@ -1021,6 +1072,18 @@ __global__ __attribute__((
 #pragma unroll
                     for (int mb = 0; mb < NB; ++mb) oacc[mb] = mfma16(vh[mb], ph[u], oacc[mb]);
                 }
+            } else if constexpr (VA > 0) {
+                constexpr int NF = 2 * NB, VN = VA < NF ? VA : NF;
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    floatx16 &a = oacc[f / 2];
+                    a = mfma16(vh_[f % VN], ph[f % 2], a);
+                    a = mfma16(vh_[f % VN], pl[f % 2], a);
+                    if constexpr (!HALF16) a = mfma16(vl_[f % VN], ph[f % 2], a);
+                    __builtin_amdgcn_sched_barrier(kSchedAlu);
+                    if (f + VN < NF) read_v(b, f + VN);
+                    __builtin_amdgcn_sched_barrier(kSchedAlu);
+                }
             } else if constexpr (HALF16) {
                 // Two products (V has no lo half); each accumulator's products in the order of
                 // the three-product form, whose third adds zeros: the same bits.
@@ -1066,6 +1129,7 @@ __global__ __attribute__((
                 prefetch(it + 1, buf ^ 1);
             if (live && tile >= my_t0 && tile <= my_t1 && tile <= c_hi) {
                 tile_qk(buf, sacc);
+                preread_v(buf);
                 tile_softmax(buf, tile * kTile, sacc, ph, pl);
                 // The P V products at raised wave priority: with two waves on a SIMD, the one
                 // that reaches them issues first, so that the other's softmax runs beside
