@@ -9,9 +9,10 @@
 // Two regimes:
 //  - Few rows (decode, m <= kLinearGemvRows): HBM-bound on the weight (2*in*out bytes per
 //    launch). One wave per kRowsPerWave output features (one per wave below 16384
-//    features); lanes stride the contraction in 16-byte chunks (8 halves), each chunk
-//    reused for every x row; the multiply-adds read the halves directly (v_fma_mix_f32)
-//    and accumulate in f32. A wave reduction ends it.
+//    features), or, for long rows, a workgroup per 4 or 8 features; lanes stride the
+//    contraction in 16-byte chunks (8 halves), each chunk reused for every x row; the
+//    multiply-adds read the halves directly (v_fma_mix_f32) and accumulate in f32. A wave
+//    reduction (and a sum of the four waves) ends it.
 //  - Many rows (prefill): matrix cores. The weight is exactly representable in f16, so
 //    only x needs care: each x row is scaled by a power of two 2^-e (its largest
 //    magnitude lands in [2^14, 2^15)) and split into x_hi = f16(x') and
@@ -77,25 +78,21 @@ __device__ __forceinline__ float wave_sum(float v) {
 constexpr int kRowsPerWave = 4;   // output features per wave
 // Fewer output features than this many waves' worth (at kRowsPerWave each, i.e. below
 // 16384 features) run one feature per wave, so that the launch still spreads over the
-// chip: the Qwen o_proj (1024 features, in 2048) is 64 workgroups at four features per
-// wave and 256 at one. A feature's sum is the same either way (the same lanes, chunks and
-// reduction), so the results are bit-identical. Measured (us per launch, 64 launches per
-// graph, one box; four -> one feature per wave): Qwen o_proj 3.45 -> 2.53, q_proj 2.85 ->
-// 2.28, k/v_proj 2.82 -> 2.19, o_proj at 4 rows 6.63 -> 4.50, Mistral k_proj 4.66 -> 3.22,
-// o_proj 8.42 -> 8.14, fused q/k/v (6144 features) 10.9 -> 10.5, a 4096-row head 3.08 ->
-// 2.86. The Qwen LM head (151936 features) keeps four: one measured 44.1 -> 72.0, and
-// two / eight 50.6 / 47.9 against four's 43.5 (the Mistral head, 32768 x 4096: 41.0 / 60.8
-// against 39.6).
+// chip. A feature's sum is the same either way (the same lanes, chunks and reduction), so
+// the results are bit-identical. Measured (us per launch, 64 launches per graph, one box;
+// four -> one feature per wave): Qwen q_proj 2.85 -> 2.28, k/v_proj 2.82 -> 2.19, a 4096-row
+// head 3.08 -> 2.86. The Qwen LM head (151936 features) keeps four: one measured 44.1 ->
+// 72.0, and two / eight 50.6 / 47.9 against four's 43.5.
 #ifndef EB_GEMV_ONE_ROW_UNITS
 #define EB_GEMV_ONE_ROW_UNITS 4096
 #endif
 constexpr int kGemvOneRowUnits = EB_GEMV_ONE_ROW_UNITS;
-// 16-byte weight chunks per lane in flight per feature. Rows of up to 1024 halves take one
-// per pass: the Qwen LM head (in 1024) read at 5.0 TB/s with 4 (half of them clamped
-// repeats of the row's last chunk), 6.3 TB/s with 2 and 6.9 TB/s with 1; 8 features per
-// wave at 1 or 2 chunks measured 6.1-6.3. Longer rows keep 4: at in 4096 (the Mistral LM
-// head) 4 chunks read 6.39 TB/s, 2 chunks 5.93 and 1 chunk 6.22.
-constexpr int gemv_unroll(int k) { return k <= 1024 ? 1 : 4; }
+// Rows of up to this many halves are one wave's, a 16-byte chunk per lane and feature at a time:
+// the Qwen LM head (in 1024) read at 5.0 TB/s with 4 chunks in flight (half of them clamped
+// repeats of the row's last chunk), 6.3 TB/s with 2 and 6.9 TB/s with 1; 8 features per wave at 1
+// or 2 chunks measured 6.1-6.3. Longer rows keep 4 chunks where they keep this kernel (many
+// features, 3 to 8 rows), or are linear_gemv_long_kernel's.
+constexpr int kGemvShortRow = 1024;
 
 // MR: capacity in x rows (the launch passes m <= MR). Requires in % 8 == 0 and 16-byte
 // aligned x, w and rows (in % 8 == 0 keeps every row start aligned).
@@ -179,6 +176,90 @@ void launch_gemv(unsigned blocks, hipStream_t st, const float *x, const LinearSe
         linear_gemv_kernel<4, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
     else
         linear_gemv_kernel<(int)eb::kLinearGemvRows, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+}
+
+// Rows of more than kGemvShortRow halves: the workgroup's four waves share F features, thread t
+// taking chunks t, t + 256, ... of every row; the waves' sums meet in LDS. What bound the
+// one-wave-per-row form was not the weight but x, which every wave read whole (16 KB for 8 KB of
+// weights at in 4096); here a wave reads a quarter of it for F features, and a thread has F loads
+// of 16 bytes in flight. Measured (us, launches in a layer or a head): Mistral token at 6000 keys
+// 31.5 -> 29.1, Mistral 8 rows 78.4 -> 60.0, Qwen 8 rows 44.2 -> 35.5 (F 4; F 8 29.3, 62.6, 38.2;
+// two chunks a pass 29.3 with F 4, 32.6 with F 8). Weights of 16384 features and more take F 8:
+// 2560 x 60000 at 2 rows 68.1 -> 51.0 (F 4 54.6), 1536 x 100000 54.3 -> 48.6 (48.3), 4096 x 32768
+// 44.7 -> 43.1 (43.8), F 16 up to 1.15 times slower; from 3 rows on, whose x is most of the
+// traffic again, they keep four features per wave (1152 x 130208 at 8 rows 192.8, F 4 200.6, F 8 241).
+// The sums are shorter chains than a wave's of the whole row.
+template <int MR, int F>
+__global__ __launch_bounds__(kThreads) void linear_gemv_long_kernel(const float *__restrict__ x,
+                                                                    LinearSegs s, int m, int K) {
+    __shared__ float part[kWaves][F * MR];
+    const int tid = threadIdx.x;
+    const int sg = seg_of(s, blockIdx.x);
+    const int N = s.n[sg];
+    const int o0 = (blockIdx.x - s.first[sg]) * F;
+    const _Float16 *w = s.w[sg];
+    const int k8 = K / 8;
+
+    float acc[F][MR];
+#pragma unroll
+    for (int r = 0; r < F; ++r)
+#pragma unroll
+        for (int i = 0; i < MR; ++i) acc[r][i] = 0.0f;
+
+    for (int c = tid; c < k8; c += kThreads) {
+        f16x8 wv[F];  // (non-temporal as above; features past the last repeat it)
+#pragma unroll
+        for (int r = 0; r < F; ++r)
+            wv[r] = __builtin_nontemporal_load(reinterpret_cast<const f16x8 *>(
+                w + (size_t)min(o0 + r, N - 1) * K + (size_t)c * 8));
+#pragma unroll
+        for (int i = 0; i < MR; ++i) {
+            if (i >= m) break;
+            const f32x4 xa = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8);
+            const f32x4 xb = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8 + 4);
+#pragma unroll
+            for (int r = 0; r < F; ++r) {
+                const f16x8 h = wv[r];
+                float t = acc[r][i];
+                t += xa.x * (float)h[0];
+                t += xa.y * (float)h[1];
+                t += xa.z * (float)h[2];
+                t += xa.w * (float)h[3];
+                t += xb.x * (float)h[4];
+                t += xb.y * (float)h[5];
+                t += xb.z * (float)h[6];
+                t += xb.w * (float)h[7];
+                acc[r][i] = t;
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < F; ++r)
+#pragma unroll
+        for (int i = 0; i < MR; ++i) {
+            const float v = wave_sum(acc[r][i]);
+            if ((tid & 63) == 0) part[tid >> 6][r * MR + i] = v;
+        }
+    __syncthreads();
+    if (tid >= F * MR) return;
+    const int r = tid / MR, i = tid % MR;
+    if (i < m && o0 + r < N)
+        s.y[sg][(size_t)i * N + o0 + r] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
+}
+
+template <int F>
+void launch_gemv_long(unsigned blocks, hipStream_t st, const float *x, const LinearSegs &s, int m,
+                      int K) {
+    if (m <= 1)
+        linear_gemv_long_kernel<1, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+    else if (m <= 2)
+        linear_gemv_long_kernel<2, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+    else if constexpr (F <= 4) {
+        if (m <= 4)
+            linear_gemv_long_kernel<4, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+        else
+            linear_gemv_long_kernel<(int)eb::kLinearGemvRows, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+    }
 }
 
 // ---------------------------------------------------------------- any shape -----------
@@ -932,20 +1013,18 @@ eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_
     if (m <= kLinearGemvRows) {
         size_t units4 = 0;
         for (int i = 0; i < nseg; ++i) units4 += (out_f[i] + kRowsPerWave - 1) / kRowsPerWave;
-        const int rpw = units4 < (size_t)kGemvOneRowUnits ? 1 : kRowsPerWave;
+        const bool few = units4 < (size_t)kGemvOneRowUnits, longer = in_f > (size_t)kGemvShortRow;
+        const bool split = longer && (few || m <= 2);  // (linear_gemv_long_kernel)
+        const size_t per = split ? (few ? 4 : 8) : (few ? 1 : kRowsPerWave);  // features per unit
         s.first[0] = 0;
-        for (int i = 0; i < nseg; ++i)
-            s.first[i + 1] = s.first[i] + (int)((out_f[i] + rpw - 1) / rpw);
-        const unsigned blocks = (unsigned)((s.first[nseg] + kWaves - 1) / kWaves);
-        const int mi = (int)m;
-        const bool one = gemv_unroll((int)in_f) == 1;
-        if (rpw == 1) {
-            if (one) launch_gemv<1, 1>(blocks, st, x, s, mi, (int)in_f);
-            else launch_gemv<4, 1>(blocks, st, x, s, mi, (int)in_f);
-        } else {
-            if (one) launch_gemv<1, kRowsPerWave>(blocks, st, x, s, mi, (int)in_f);
-            else launch_gemv<4, kRowsPerWave>(blocks, st, x, s, mi, (int)in_f);
-        }
+        for (int i = 0; i < nseg; ++i) s.first[i + 1] = s.first[i] + (int)((out_f[i] + per - 1) / per);
+        const unsigned units = (unsigned)s.first[nseg], blocks = (units + kWaves - 1) / kWaves;
+        const int mi = (int)m, k = (int)in_f;
+        if (split && few) launch_gemv_long<4>(units, st, x, s, mi, k);
+        else if (split) launch_gemv_long<8>(units, st, x, s, mi, k);
+        else if (few) launch_gemv<1, 1>(blocks, st, x, s, mi, k);
+        else if (longer) launch_gemv<4, kRowsPerWave>(blocks, st, x, s, mi, k);
+        else launch_gemv<1, kRowsPerWave>(blocks, st, x, s, mi, k);
         return check_launch("linear_f16w");
     }
     if (ws == nullptr || ws_floats < m) return fail(EB_SHAPE_MISMATCH, "linear: workspace too small");

@@ -189,6 +189,24 @@ def test_gemv_features_per_wave_same_bits(dev, m):
     assert_close(got_small, want_of(x, w[:small], m, in_f, small), what="gemv one per wave")
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4, 5, 8])
+@pytest.mark.parametrize("in_f,out_f", [
+    (1032, 1), (1536, 7), (2048, 1024), (2056, 9), (4096, 61), (6152, 12),  # 4 features a workgroup
+    (1032, 16384), (1800, 16391),   # 8 (or, from 3 rows on, four a wave)
+])
+def test_long_rows_match_oracle(dev, m, in_f, out_f):
+    """Contractions past 1024: rows shared by a workgroup's waves, with part of a pass (1032,
+    1536, 1800), one pass, and one chunk more; features on and past the workgroup's 4 or 8."""
+    note(f"linear gemv long rows m={m} in={in_f} out={out_f}")
+    x = oracle.randn((m, in_f), 41)
+    w = oracle.randn((out_f, in_f), 42) * np.float32(in_f ** -0.5)
+    got = run(dev, x, w, m, in_f, out_f)
+    cols = sorted({c for c in (*range(0, 40), *range(out_f - 40, out_f)) if 0 <= c < out_f})
+    want = want_of(x, np.ascontiguousarray(w[cols]), m, in_f, len(cols))
+    assert np.isfinite(got).all()
+    assert_close(got[:, cols], want, what="long rows")
+
+
 def test_raw_launch_with_workspace(dev):
     note("linear raw launch")
     m, in_f, out_f = 50, 1024, 320
