@@ -68,6 +68,10 @@ __device__ __forceinline__ SegView seg_of(const eb::RowsArgs &a, int t) {
     return v;
 }
 
+// All loads of a row (its values, gain and angles) go out before its sum is formed: with the gain
+// and angles after it, a row took two memory latencies. Gemma-4 (us, whole call): 1000 rows into
+// E4M3 71.8 -> 69.6, 500 rows 44.6 -> 43.7, 2000 rows 177.8 -> 176.5 (two rows per lane 177.3).
+// Bound by HBM beyond that: 131 MB in 22 us at 2000 rows.
 template <int LPR>
 __global__ __launch_bounds__(kThreads) void rows_vec_kernel(eb::RowsArgs a) {
 #pragma clang fp contract(off)
@@ -83,9 +87,22 @@ __global__ __launch_bounds__(kThreads) void rows_vec_kernel(eb::RowsArgs a) {
     const int tok = sv.local / sv.nh;
     const int hh = sv.local % sv.nh;
     const f32x4 z = {0.f, 0.f, 0.f, 0.f};
-    const float *src = sv.src + ((size_t)tok * sv.nh + hh) * hd + 4 * j;
-    f32x4 x1 = on ? *reinterpret_cast<const f32x4 *>(src) : z;
-    f32x4 x2 = on ? *reinterpret_cast<const f32x4 *>(src + half) : z;
+    const int jj = j < hd / 8 ? 4 * j : 0;  // (lanes past the row read its start)
+    const float *src = sv.src + ((size_t)tok * sv.nh + hh) * hd + jj;
+    f32x4 x1 = *reinterpret_cast<const f32x4 *>(src);
+    f32x4 x2 = *reinterpret_cast<const f32x4 *>(src + half);
+    f32x4 g1, g2, c, s;
+    if (sv.gain) {
+        g1 = *reinterpret_cast<const f32x4 *>(sv.gain + jj);
+        g2 = *reinterpret_cast<const f32x4 *>(sv.gain + half + jj);
+    }
+    if (sv.rope) {
+        const size_t trow = (size_t)(a.rope_row0 + tok) * half + jj;
+        c = *reinterpret_cast<const f32x4 *>(a.cosb + trow);
+        s = *reinterpret_cast<const f32x4 *>(a.sinb + trow);
+    }
+    x1 = on ? x1 : z;
+    x2 = on ? x2 : z;
     // Every lane joins the reduction (rows of one group share their segment).
     float ss = (x1.x * x1.x + x1.y * x1.y) + (x1.z * x1.z + x1.w * x1.w) +
                ((x2.x * x2.x + x2.y * x2.y) + (x2.z * x2.z + x2.w * x2.w));
@@ -93,13 +110,10 @@ __global__ __launch_bounds__(kThreads) void rows_vec_kernel(eb::RowsArgs a) {
     if (!on) return;
     if (sv.gain) {
         const float inv = 1.0f / sqrtf(ss / (float)hd + a.eps);
-        x1 = x1 * inv * *reinterpret_cast<const f32x4 *>(sv.gain + 4 * j);
-        x2 = x2 * inv * *reinterpret_cast<const f32x4 *>(sv.gain + half + 4 * j);
+        x1 = x1 * inv * g1;
+        x2 = x2 * inv * g2;
     }
     if (sv.rope) {
-        const size_t trow = (size_t)(a.rope_row0 + tok) * half + 4 * j;
-        const f32x4 c = *reinterpret_cast<const f32x4 *>(a.cosb + trow);
-        const f32x4 s = *reinterpret_cast<const f32x4 *>(a.sinb + trow);
         const f32x4 y1 = x1 * c - x2 * s;
         const f32x4 y2 = x2 * c + x1 * s;
         x1 = y1;
