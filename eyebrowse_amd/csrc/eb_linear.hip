@@ -726,7 +726,8 @@ linear_tile_kernel(const _Float16 *__restrict__ xs, const float *__restrict__ ex
             const void *base = b >= 2 * BM * ROWB / 1024 ? static_cast<const void *>(w)
                                                          : static_cast<const void *>(xs);
             const unsigned dst = __builtin_amdgcn_readfirstlane(lds0 + buf * C::STAGE + b * 1024);
-            asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+            // (s_nop: a copy to LDS may read m0 one wait state after its write at the soonest.)
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                          :
                          : "s"(dst), "v"(voff[i]), "s"(base)
                          : "memory", "m0");

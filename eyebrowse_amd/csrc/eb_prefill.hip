@@ -450,7 +450,7 @@ __device__ __forceinline__ void img_copy(const float *__restrict__ recs, float *
 #pragma unroll
         for (int i = 0; i < BPW; ++i) {
             if (BLK % NW == 0 || j0 + i < BLK)  // (uniform)
-                asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, off offset:%2"
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2"
                              :
                              : "s"(dst + 4096 * (i / 4)), "v"(src + 1024 * (i / 4)),
                                "i"(1024 * (i % 4))
