@@ -399,7 +399,8 @@ eb_status eb_linear_f16w_multi(eb_recorder *rec, const eb_tensor *a, size_t n,
                                const size_t *out_f, size_t m, size_t in_f);
 /* Raw form: w holds w_halves IEEE halves (the packed words read as uint16_t). Rows m > 8
  * need eb_linear_workspace_floats(m, in_f) floats of workspace (row exponents; no
- * initialisation needed). */
+ * initialisation needed). With a 16-byte aligned workspace of m rounded up to 64, plus
+ * m * in_f floats, and in_f a multiple of 64, the rows are split once into it (faster). */
 size_t eb_linear_workspace_floats(size_t m, size_t in_f);
 eb_status eb_launch_linear_f16w(void *stream, const float *a, size_t a_numel, const uint16_t *w,
                                 size_t w_halves, float *c, size_t c_numel, size_t m, size_t in_f,
