@@ -423,38 +423,61 @@ __device__ __forceinline__ void prefill_store_step(float *smem, const f32x4 (&rk
     }
 }
 
+// N (1 to 4) KiB from src (this lane's 16 bytes of the first) to LDS byte address dst, which m0
+// holds for all of them: a load's immediate offset applies to both its global and its LDS
+// address. A wait state follows the write of m0 (a copy to LDS may read it one after at the
+// soonest; inside an asm block the compiler adds none).
+#define EB_LDS_COPY_1 "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+#define EB_LDS_COPY_2 EB_LDS_COPY_1 "\n\tglobal_load_lds_dwordx4 %1, off offset:1024"
+#define EB_LDS_COPY_3 EB_LDS_COPY_2 "\n\tglobal_load_lds_dwordx4 %1, off offset:2048"
+#define EB_LDS_COPY_4 EB_LDS_COPY_3 "\n\tglobal_load_lds_dwordx4 %1, off offset:3072"
+template <int N>
+__device__ __forceinline__ void lds_copy_kib(unsigned dst, const float *src) {
+    static_assert(N >= 1 && N <= 4, "immediate offsets end at 4095");
+    if constexpr (N == 1) asm volatile(EB_LDS_COPY_1 : : "s"(dst), "v"(src) : "memory", "m0");
+    if constexpr (N == 2) asm volatile(EB_LDS_COPY_2 : : "s"(dst), "v"(src) : "memory", "m0");
+    if constexpr (N == 3) asm volatile(EB_LDS_COPY_3 : : "s"(dst), "v"(src) : "memory", "m0");
+    if constexpr (N == 4) asm volatile(EB_LDS_COPY_4 : : "s"(dst), "v"(src) : "memory", "m0");
+}
+#undef EB_LDS_COPY_4
+#undef EB_LDS_COPY_3
+#undef EB_LDS_COPY_2
+#undef EB_LDS_COPY_1
+
 // Copy NIMG tile images (records tile0 .. tile0 + NIMG - 1 of one KV head, recs, each
 // clamped to the last record, nt - 1: a clamped image is never read) of IMGF floats into
 // LDS at lds with memory-to-LDS loads: wave w moves KiB blocks w * BPW .. w * BPW + BPW - 1
-// of each image (lane i bytes 16i .. 16i + 15 of a block), a load's immediate offset
-// applying to both its global and its LDS address. Issued as inline assembly, which the
-// compiler's wait counting does not see (it would otherwise wait for these loads before
-// every read of the other buffer); the loads are complete after wait_vm_all(). m0 is a
-// reserved register, so the compiler warns that it does not preserve it around the asm:
-// the generated code of these kernels keeps no value of its own in m0 (in their gfx950
-// assembly every m0 write is this asm's), so nothing else sees the clobber.
+// of each image, and block NW * BPW + w of those left over (lane i bytes 16i .. 16i + 15 of a
+// block). Issued as inline assembly, which the compiler's wait counting does not see (it would
+// otherwise wait for these loads before every read of the other buffer); the loads are complete
+// after wait_vm_all(). m0 is a reserved register, so the compiler warns that it does not
+// preserve it around the asm: the generated code of these kernels keeps no value of its own in
+// m0 (in their gfx950 assembly every m0 write is this asm's), so nothing else sees the clobber.
+// Against a write and a wait per block (us): f16 mode, Mistral 3001 rows 108.3 -> 106.3, 4096
+// 172.4 -> 170.3, Qwen 1000 28.0 -> 27.7; the accurate mode, which issues more beside the
+// copies, is unchanged (Mistral 2000 119.2 -> 118.5, Gemma-4 2000 157.6 -> 156.9).
 template <int IMGF, int NIMG, int NW>
 __device__ __forceinline__ void img_copy(const float *__restrict__ recs, float *lds, int tile0,
                                          int nt, int wave, int lane) {
     constexpr int BLK = IMGF / 256;  // KiB blocks per image
-    constexpr int BPW = (BLK + NW - 1) / NW;
+    constexpr int BPW = BLK / NW, REST = BLK % NW;
     static_assert(IMGF % 256 == 0, "whole KiB images");
-    const int j0 = wave * BPW;
 #pragma unroll
     for (int k = 0; k < NIMG; ++k) {
         const int t = min(tile0 + k, nt - 1);
-        const float *src = recs + (size_t)t * IMGF + j0 * 256 + lane * 4;
-        const unsigned dst = __builtin_amdgcn_readfirstlane(
-            (unsigned)(uintptr_t)(__attribute__((address_space(3))) float *)(lds + k * IMGF +
-                                                                              j0 * 256));
+        const float *src = recs + (size_t)t * IMGF + lane * 4;
+        const unsigned dst = (unsigned)(uintptr_t)(__attribute__((address_space(3))) float *)(
+            lds + k * IMGF);
+        const int j0 = wave * BPW;
+        const unsigned d0 = __builtin_amdgcn_readfirstlane(dst + 1024 * j0);
 #pragma unroll
-        for (int i = 0; i < BPW; ++i) {
-            if (BLK % NW == 0 || j0 + i < BLK)  // (uniform)
-                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off offset:%2"
-                             :
-                             : "s"(dst + 4096 * (i / 4)), "v"(src + 1024 * (i / 4)),
-                               "i"(1024 * (i % 4))
-                             : "memory", "m0");
+        for (int i = 0; i < BPW / 4; ++i) lds_copy_kib<4>(d0 + 4096 * i, src + 256 * j0 + 1024 * i);
+        if constexpr (BPW % 4 > 0)
+            lds_copy_kib<BPW % 4>(d0 + 1024 * (BPW / 4 * 4), src + 256 * j0 + 256 * (BPW / 4 * 4));
+        if constexpr (REST > 0) {
+            const int j = NW * BPW + wave;
+            if (wave < REST)  // (uniform)
+                lds_copy_kib<1>(__builtin_amdgcn_readfirstlane(dst + 1024 * j), src + 256 * j);
         }
     }
 }
