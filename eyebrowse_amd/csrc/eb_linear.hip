@@ -90,13 +90,12 @@ constexpr int kGemvOneRowUnits = EB_GEMV_ONE_ROW_UNITS;
 // Rows of up to this many halves are one wave's, a 16-byte chunk per lane and feature at a time:
 // the Qwen LM head (in 1024) read at 5.0 TB/s with 4 chunks in flight (half of them clamped
 // repeats of the row's last chunk), 6.3 TB/s with 2 and 6.9 TB/s with 1; 8 features per wave at 1
-// or 2 chunks measured 6.1-6.3. Longer rows keep 4 chunks where they keep this kernel (many
-// features, 3 to 8 rows), or are linear_gemv_long_kernel's.
+// or 2 chunks measured 6.1-6.3. Longer rows are linear_gemv_long_kernel's.
 constexpr int kGemvShortRow = 1024;
 
 // MR: capacity in x rows (the launch passes m <= MR). Requires in % 8 == 0 and 16-byte
 // aligned x, w and rows (in % 8 == 0 keeps every row start aligned).
-template <int MR, int kChunkUnroll, int RPW = kRowsPerWave>
+template <int MR, int RPW>
 __global__ __launch_bounds__(kThreads) void linear_gemv_kernel(const float *__restrict__ x,
                                                                LinearSegs s, int m, int K) {
     const int lane = threadIdx.x & 63;
@@ -115,44 +114,37 @@ __global__ __launch_bounds__(kThreads) void linear_gemv_kernel(const float *__re
 #pragma unroll
         for (int i = 0; i < MR; ++i) acc[r][i] = 0.0f;
 
-    for (int c0 = 0; c0 < k8; c0 += 64 * kChunkUnroll) {
+    for (int c0 = 0; c0 < k8; c0 += 64) {
         // All weight loads of the step first (clamped addresses, masked values), non-temporal:
         // each weight is read once per launch (the Qwen LM head, 311 MB: 4.78 -> 5.07 TB/s).
-        f16x8 wv[kChunkUnroll][RPW];
+        f16x8 wv[RPW];
+        const int c = c0 + lane;
+        const int cc = c < k8 ? c : k8 - 1;
 #pragma unroll
-        for (int u = 0; u < kChunkUnroll; ++u) {
-            const int c = c0 + u * 64 + lane;
-            const int cc = c < k8 ? c : k8 - 1;
+        for (int r = 0; r < RPW; ++r) {
+            const int o = min(o0 + r, N - 1);
+            wv[r] = __builtin_nontemporal_load(
+                reinterpret_cast<const f16x8 *>(w + (size_t)o * K + (size_t)cc * 8));
+        }
+        if (c >= k8) break;
+#pragma unroll
+        for (int i = 0; i < MR; ++i) {
+            if (i >= m) break;
+            const f32x4 xa = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8);
+            const f32x4 xb = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8 + 4);
 #pragma unroll
             for (int r = 0; r < RPW; ++r) {
-                const int o = min(o0 + r, N - 1);
-                wv[u][r] = __builtin_nontemporal_load(
-                    reinterpret_cast<const f16x8 *>(w + (size_t)o * K + (size_t)cc * 8));
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kChunkUnroll; ++u) {
-            const int c = c0 + u * 64 + lane;
-            if (c >= k8) break;
-#pragma unroll
-            for (int i = 0; i < MR; ++i) {
-                if (i >= m) break;
-                const f32x4 xa = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8);
-                const f32x4 xb = *reinterpret_cast<const f32x4 *>(x + (size_t)i * K + c * 8 + 4);
-#pragma unroll
-                for (int r = 0; r < RPW; ++r) {
-                    const f16x8 h = wv[u][r];
-                    float t = acc[r][i];
-                    t += xa.x * (float)h[0];
-                    t += xa.y * (float)h[1];
-                    t += xa.z * (float)h[2];
-                    t += xa.w * (float)h[3];
-                    t += xb.x * (float)h[4];
-                    t += xb.y * (float)h[5];
-                    t += xb.z * (float)h[6];
-                    t += xb.w * (float)h[7];
-                    acc[r][i] = t;
-                }
+                const f16x8 h = wv[r];
+                float t = acc[r][i];
+                t += xa.x * (float)h[0];
+                t += xa.y * (float)h[1];
+                t += xa.z * (float)h[2];
+                t += xa.w * (float)h[3];
+                t += xb.x * (float)h[4];
+                t += xb.y * (float)h[5];
+                t += xb.z * (float)h[6];
+                t += xb.w * (float)h[7];
+                acc[r][i] = t;
             }
         }
     }
@@ -165,35 +157,40 @@ __global__ __launch_bounds__(kThreads) void linear_gemv_kernel(const float *__re
         }
 }
 
-template <int U, int RPW>
+template <int RPW>
 void launch_gemv(unsigned blocks, hipStream_t st, const float *x, const LinearSegs &s, int m,
                  int K) {
     if (m <= 1)
-        linear_gemv_kernel<1, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+        linear_gemv_kernel<1, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
     else if (m <= 2)
-        linear_gemv_kernel<2, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+        linear_gemv_kernel<2, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
     else if (m <= 4)
-        linear_gemv_kernel<4, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+        linear_gemv_kernel<4, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
     else
-        linear_gemv_kernel<(int)eb::kLinearGemvRows, U, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+        linear_gemv_kernel<(int)eb::kLinearGemvRows, RPW><<<blocks, kThreads, 0, st>>>(x, s, m, K);
 }
 
 // Rows of more than kGemvShortRow halves: the workgroup's four waves share F features, thread t
-// taking chunks t, t + 256, ... of every row; the waves' sums meet in LDS. What bound the
+// taking chunks t, t + 256, ... of every row. The threads' sums meet in LDS, where thread l of a
+// wave adds those of threads l, 64 + l, 128 + l and 192 + l before the wave's sum: one wave sum
+// per value, where one in each wave cost 8 rows over 100000 features 5 %. What bounded the
 // one-wave-per-row form was not the weight but x, which every wave read whole (16 KB for 8 KB of
 // weights at in 4096); here a wave reads a quarter of it for F features, and a thread has F loads
-// of 16 bytes in flight. Measured (us, launches in a layer or a head): Mistral token at 6000 keys
-// 31.5 -> 29.1, Mistral 8 rows 78.4 -> 60.0, Qwen 8 rows 44.2 -> 35.5 (F 4; F 8 29.3, 62.6, 38.2;
-// two chunks a pass 29.3 with F 4, 32.6 with F 8). Weights of 16384 features and more take F 8:
-// 2560 x 60000 at 2 rows 68.1 -> 51.0 (F 4 54.6), 1536 x 100000 54.3 -> 48.6 (48.3), 4096 x 32768
-// 44.7 -> 43.1 (43.8), F 16 up to 1.15 times slower; from 3 rows on, whose x is most of the
-// traffic again, they keep four features per wave (1152 x 130208 at 8 rows 192.8, F 4 200.6, F 8 241).
-// The sums are shorter chains than a wave's of the whole row.
+// of 16 bytes in flight. Measured (us, launches in a layer or a head, one wave per row or per four
+// -> this form): Mistral token at 6000 keys 31.5 -> 29.0, Mistral 8 rows 78.4 -> 59.8, Qwen 8 rows
+// 44.2 -> 35.5 (F 4; F 8 0.2 to 8 % slower). Weights of 16384 features and more: 2560 x 60000 at 2
+// rows 68.1 -> 51.9, 3 rows 78.2 -> 74.2, 8 rows 135.4 -> 138.3; 4096 x 32768 at 4 rows 64.9 ->
+// 59.6, 8 rows 96.5 -> 92.6; 1152 x 130000, where a row is 144 chunks for 256 threads, 3 rows 92.9
+// -> 94.5, 8 rows 193.4 -> 193.3. Those take F 8 up to 4 rows (1 row 2560 x 60000 49.6, F 4 54.6;
+// 4 rows 80.7, F 4 87.3), F 4 from 5 on (8 rows 138.4, F 8 148.2: the registers leave two waves
+// per SIMD).
+// The order of a sum depends on K alone (here, and above for K up to kGemvShortRow): not on the
+// rows of the call, on F, or on the launch's other outputs.
 template <int MR, int F>
 __global__ __launch_bounds__(kThreads) void linear_gemv_long_kernel(const float *__restrict__ x,
                                                                     LinearSegs s, int m, int K) {
-    __shared__ float part[kWaves][F * MR];
-    const int tid = threadIdx.x;
+    __shared__ float part[F * MR][kThreads];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sg = seg_of(s, blockIdx.x);
     const int N = s.n[sg];
     const int o0 = (blockIdx.x - s.first[sg]) * F;
@@ -236,15 +233,17 @@ __global__ __launch_bounds__(kThreads) void linear_gemv_long_kernel(const float 
 #pragma unroll
     for (int r = 0; r < F; ++r)
 #pragma unroll
-        for (int i = 0; i < MR; ++i) {
-            const float v = wave_sum(acc[r][i]);
-            if ((tid & 63) == 0) part[tid >> 6][r * MR + i] = v;
-        }
+        for (int i = 0; i < MR; ++i)
+            if (i < m) part[r * MR + i][tid] = acc[r][i];
     __syncthreads();
-    if (tid >= F * MR) return;
-    const int r = tid / MR, i = tid % MR;
-    if (i < m && o0 + r < N)
-        s.y[sg][(size_t)i * N + o0 + r] = (part[0][tid] + part[1][tid]) + (part[2][tid] + part[3][tid]);
+#pragma unroll
+    for (int v = 0; v < F * MR / kWaves; ++v) {
+        const int f = v * kWaves + wave;
+        if (f % MR >= m) continue;
+        const float t = (part[f][lane] + part[f][64 + lane]) + (part[f][128 + lane] + part[f][192 + lane]);
+        const float sum = wave_sum(t);
+        if (lane == 0 && o0 + f / MR < N) s.y[sg][(size_t)(f % MR) * N + o0 + f / MR] = sum;
+    }
 }
 
 template <int F>
@@ -254,12 +253,12 @@ void launch_gemv_long(unsigned blocks, hipStream_t st, const float *x, const Lin
         linear_gemv_long_kernel<1, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
     else if (m <= 2)
         linear_gemv_long_kernel<2, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
-    else if constexpr (F <= 4) {
-        if (m <= 4)
-            linear_gemv_long_kernel<4, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
-        else
-            linear_gemv_long_kernel<(int)eb::kLinearGemvRows, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
-    }
+    else if (m <= 3)
+        linear_gemv_long_kernel<3, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+    else if (m <= 4 || F > 4)  // (F 8 takes up to 4 rows)
+        linear_gemv_long_kernel<4, F><<<blocks, kThreads, 0, st>>>(x, s, m, K);
+    else
+        linear_gemv_long_kernel<(int)eb::kLinearGemvRows, 4><<<blocks, kThreads, 0, st>>>(x, s, m, K);
 }
 
 // ---------------------------------------------------------------- any shape -----------
@@ -1023,17 +1022,16 @@ eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_
         size_t units4 = 0;
         for (int i = 0; i < nseg; ++i) units4 += (out_f[i] + kRowsPerWave - 1) / kRowsPerWave;
         const bool few = units4 < (size_t)kGemvOneRowUnits, longer = in_f > (size_t)kGemvShortRow;
-        const bool split = longer && (few || m <= 2);  // (linear_gemv_long_kernel)
-        const size_t per = split ? (few ? 4 : 8) : (few ? 1 : kRowsPerWave);  // features per unit
+        // Features per unit: a workgroup's (longer rows) or a wave's.
+        const size_t per = longer ? (few || m > 4 ? 4 : 8) : (few ? 1 : kRowsPerWave);
         s.first[0] = 0;
         for (int i = 0; i < nseg; ++i) s.first[i + 1] = s.first[i] + (int)((out_f[i] + per - 1) / per);
         const unsigned units = (unsigned)s.first[nseg], blocks = (units + kWaves - 1) / kWaves;
         const int mi = (int)m, k = (int)in_f;
-        if (split && few) launch_gemv_long<4>(units, st, x, s, mi, k);
-        else if (split) launch_gemv_long<8>(units, st, x, s, mi, k);
-        else if (few) launch_gemv<1, 1>(blocks, st, x, s, mi, k);
-        else if (longer) launch_gemv<4, kRowsPerWave>(blocks, st, x, s, mi, k);
-        else launch_gemv<1, kRowsPerWave>(blocks, st, x, s, mi, k);
+        if (longer && per == 4) launch_gemv_long<4>(units, st, x, s, mi, k);
+        else if (longer) launch_gemv_long<8>(units, st, x, s, mi, k);
+        else if (few) launch_gemv<1>(blocks, st, x, s, mi, k);
+        else launch_gemv<kRowsPerWave>(blocks, st, x, s, mi, k);
         return check_launch("linear_f16w");
     }
     if (ws == nullptr || ws_floats < m) return fail(EB_SHAPE_MISMATCH, "linear: workspace too small");

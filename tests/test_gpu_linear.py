@@ -271,3 +271,17 @@ def test_wide_tile_gemm_sampled_rows(dev, m, outs):
         got = cs[i].to_f32().reshape(m, o)[rows]
         want = oracle.linear_f16w(x[rows], oracle.f16_bits(ws[i]), len(rows), in_f, o, threads=16)
         assert_close(got, want, what=f"projection {i}")
+
+
+@pytest.mark.parametrize("in_f", [512, 1024, 1032, 1536, 2056, 4096])
+@pytest.mark.parametrize("out_f", [1001, 16387])
+def test_few_rows_bits_do_not_depend_on_the_call(dev, in_f, out_f):
+    """A row's results are the same bits whichever way it is called: alone, among 2 to 8 rows, for
+    a few features or for the 16384 and more that other launch shapes take."""
+    note(f"linear few rows, bits in={in_f} out={out_f}")
+    x = oracle.randn((8, in_f), 51)
+    w = oracle.randn((out_f, in_f), 52) * np.float32(in_f ** -0.5)
+    want = np.concatenate([run(dev, x[i:i + 1], w[:1001], 1, in_f, 1001) for i in range(8)])
+    for m in (1, 2, 3, 4, 5, 8):
+        got = run(dev, x[:m], w, m, in_f, out_f)
+        assert_bitwise(got[:, :1001], want[:m], f"{m} rows")
