@@ -181,6 +181,9 @@ constexpr int kLinearMaxSegs = 3;
 constexpr size_t kLinearGemvRows = 8;
 size_t linear_workspace_floats(size_t m, size_t in_f);
 size_t linear_split_workspace_floats(size_t m, size_t in_f);
+// The most that a launch on these operands makes use of (unaligned ones split no rows).
+size_t linear_usable_workspace_floats(const float *x, const uint16_t *const *w,
+                                      const size_t *out_f, int nseg, size_t m, size_t in_f);
 eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_t *const *w,
                                    float *const *y, const size_t *out_f, int nseg, size_t m,
                                    size_t in_f, float *ws, size_t ws_floats);

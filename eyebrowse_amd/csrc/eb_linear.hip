@@ -984,6 +984,18 @@ size_t linear_split_workspace_floats(size_t m, size_t in_f) {
     return tile_ex_floats(m) + m * in_f;
 }
 
+size_t linear_usable_workspace_floats(const float *x, const uint16_t *const *w,
+                                      const size_t *out_f, int nseg, size_t m, size_t in_f) {
+    bool split = aligned16(x);
+    size_t total_out = 0;
+    for (int i = 0; i < nseg; ++i) {
+        split = split && aligned16(w[i]);
+        total_out += out_f[i];
+    }
+    return split && total_out > 0 ? linear_split_workspace_floats(m, in_f)
+                                  : linear_workspace_floats(m, in_f);
+}
+
 eb_status launch_linear_f16w_multi(hipStream_t st, const float *x, const uint16_t *const *w,
                                    float *const *y, const size_t *out_f, int nseg, size_t m,
                                    size_t in_f, float *ws, size_t ws_floats) {

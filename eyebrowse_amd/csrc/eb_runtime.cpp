@@ -1054,11 +1054,11 @@ static eb_status tensor_weight(const eb_tensor *t, const char *name, eb_device *
     return EB_OK;
 }
 
-// linear_f16w over nseg weight/output pairs that share x.
-static eb_status linear_checked(hipStream_t st, const float *x, size_t xn,
-                                const uint16_t *const *w, const size_t *w_halves,
-                                float *const *y, const size_t *yn, const size_t *out_f, int nseg,
-                                size_t m, size_t in_f, float *ws, size_t wsn) {
+// The operands of linear_f16w over nseg weight/output pairs that share x, without a workspace.
+static eb_status linear_operands_checked(const float *x, size_t xn, const uint16_t *const *w,
+                                         const size_t *w_halves, float *const *y,
+                                         const size_t *yn, const size_t *out_f, int nseg,
+                                         size_t m, size_t in_f) {
     if (nseg < 1 || nseg > eb::kLinearMaxSegs)
         return fail(EB_OTHER, "linear_f16w: 1 to %d weights per launch", eb::kLinearMaxSegs);
     EB_TRY(eb::check_numel(xn, {m, in_f}, "a"));
@@ -1066,13 +1066,22 @@ static eb_status linear_checked(hipStream_t st, const float *x, size_t xn,
         EB_TRY(eb::check_numel(w_halves[i], {out_f[i], in_f}, "w"));
         EB_TRY(eb::check_numel(yn[i], {m, out_f[i]}, "c"));
     }
-    if (m == 0) return eb::ok();
+    if (m == 0) return EB_OK;
     if (in_f > 0) EB_TRY(eb::check_ptr(x, "a"));
     for (int i = 0; i < nseg; ++i) {
         if (out_f[i] == 0) continue;
         if (in_f > 0) EB_TRY(eb::check_ptr(w[i], "w"));
         EB_TRY(eb::check_ptr(y[i], "c"));
     }
+    return EB_OK;
+}
+
+static eb_status linear_checked(hipStream_t st, const float *x, size_t xn,
+                                const uint16_t *const *w, const size_t *w_halves,
+                                float *const *y, const size_t *yn, const size_t *out_f, int nseg,
+                                size_t m, size_t in_f, float *ws, size_t wsn) {
+    EB_TRY(linear_operands_checked(x, xn, w, w_halves, y, yn, out_f, nseg, m, in_f));
+    if (m == 0) return eb::ok();
     const size_t need = eb::linear_workspace_floats(m, in_f);
     if (wsn < need)
         return fail(EB_SHAPE_MISMATCH, "linear_f16w: workspace holds %zu floats, needs %zu", wsn,
@@ -1098,9 +1107,13 @@ static eb_status device_linear(eb_device *dev, const eb_tensor *a,
         yp[i] = static_cast<float *>(c[i]->ptr);
         yn[i] = eb_tensor_numel(c[i]);
     }
-    // Room for the split rows, or for the row exponents alone where the workspace cannot grow
-    // that far (during a capture, or without the memory).
-    size_t wsn = eb::linear_split_workspace_floats(m, in_f);
+    const float *x = static_cast<const float *>(a->ptr);
+    const size_t xn = eb_tensor_numel(a);
+    // (before the workspace grows: by up to m * in_f floats of a call that may be refused)
+    EB_TRY(linear_operands_checked(x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f));
+    // Room for the split rows, or for the row exponents alone where the launch does not split
+    // them or the workspace cannot grow that far (during a capture, or without the memory).
+    size_t wsn = eb::linear_usable_workspace_floats(x, wp, out_f, nseg, m, in_f);
     float *ws = nullptr;
     WsLock lk;
     if (wsn > 0) {
@@ -1115,8 +1128,7 @@ static eb_status device_linear(eb_device *dev, const eb_tensor *a,
         }
         if (st != EB_OK) return st;
     }
-    return linear_checked(dev->stream, static_cast<const float *>(a->ptr), eb_tensor_numel(a),
-                          wp, wh, yp, yn, out_f, nseg, m, in_f, ws, wsn);
+    return linear_checked(dev->stream, x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f, ws, wsn);
 }
 
 // Both caches of one layer share a dtype.

@@ -149,3 +149,40 @@ def test_sums_are_cut_in_two(dev, m, in_f, limit):
     want = x.astype(np.float64) @ w.astype(np.float64).T
     err = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert err <= limit, err
+
+
+def test_a_refused_call_leaves_the_workspace():
+    """A call whose sizes do not fit its tensors is refused before the workspace grows for it. A
+    capture shows the workspace: it takes a call whose row exponents have room, and no other."""
+    note("linear refused call")
+    dev = eb.Device.new(0)
+    x, wt = upload(dev, oracle.randn((16, 40), 1)), eb.Tensor.from_f16_packed(dev, (8, 40), oracle.randn((8, 40), 2))
+    ct = eb.Tensor.empty(dev, (16, 8))
+    rec = eb.Recorder(dev)
+    with pytest.raises(eb.ShapeMismatch):
+        eb.linear_f16w(rec, x, wt, ct, 64, 64, 8)
+    rec.submit()
+    dev.begin_capture()
+    rec = eb.Recorder(dev)
+    with pytest.raises(eb.EyebrowseError, match="would have to grow"):
+        eb.linear_f16w(rec, x, wt, ct, 16, 40, 8)
+    rec.release()
+    dev.end_capture().release()
+
+
+def test_rows_that_are_not_split_take_no_room_for_it():
+    """No outputs: nothing to launch, so no room for split rows."""
+    note("linear no outputs")
+    dev = eb.Device.new(0)
+    x = upload(dev, oracle.randn((16, 64), 1))
+    rec = eb.Recorder(dev)
+    eb.linear_f16w(rec, x, eb.Tensor.empty(dev, (0, 64), eb.DType.F16), eb.Tensor.empty(dev, (16, 0)), 16, 64, 0)
+    rec.submit()
+    wt, ct = eb.Tensor.from_f16_packed(dev, (8, 40), oracle.randn((8, 40), 2)), eb.Tensor.empty(dev, (17, 8))
+    xt = upload(dev, oracle.randn((17, 40), 3))
+    dev.begin_capture()
+    rec = eb.Recorder(dev)
+    with pytest.raises(eb.EyebrowseError, match="would have to grow"):
+        eb.linear_f16w(rec, xt, wt, ct, 17, 40, 8)
+    rec.release()
+    dev.end_capture().release()
