@@ -23,6 +23,7 @@
 #include <vector>
 
 #include "eb_internal.h"
+#include "eb_workspace.h"
 
 // ------------------------------------------------------------------ errors ---------------
 
@@ -150,13 +151,9 @@ struct eb_device {
     std::mutex pool_mu;
     std::unordered_map<size_t, std::vector<void *>> pool;  // exact byte size -> free buffers
     std::mutex ws_mu;
-    float *ws = nullptr;  // split / pre-split / partials workspace, grow-only, stream ordered
-    size_t ws_floats = 0;
-    // Graphs whose kernels were captured with a workspace buffer in their arguments keep
-    // that buffer alive: live graph references per buffer, and buffers the workspace has
-    // outgrown that a graph still references (freed with the last such graph). ws_mu.
-    std::unordered_map<float *, int> ws_graph_refs;
-    std::vector<float *> ws_retired;
+    // Split / pre-split / partials workspace, grow-only, stream ordered. Graphs whose kernels
+    // were captured with a buffer of it in their arguments keep that buffer alive. ws_mu.
+    eb::Workspace ws;
     bool ws_in_capture = false;  // the running capture handed out the current workspace
     std::atomic<bool> capturing{false};  // the stream is being captured into a graph
     std::vector<Parked> parked;          // buffers released during the capture (pool_mu)
@@ -184,6 +181,25 @@ struct eb_recorder {
     bool deferred = false;  // its work is a capture of the device stream, run at submit
 };
 
+// A workspace's memory (eb_workspace.h).
+struct WorkspaceMem {
+    eb_device *dev;
+    eb_status alloc(size_t floats, float **p) {
+        const hipError_t e = hipMalloc((void **)p, floats * sizeof(float));
+        if (e == hipSuccess) return EB_OK;
+        (void)hipGetLastError();  // (reported here, and by no later call)
+        return eb::hip_fail(e, "hipMalloc (workspace)");
+    }
+    eb_status drain() {
+        EB_HIP_TRY(hipStreamSynchronize(dev->stream));
+        return EB_OK;
+    }
+    eb_status free(float *p) {
+        EB_HIP_TRY(hipFree(p));
+        return EB_OK;
+    }
+};
+
 static eb_status not_capturing(const eb_device *d, const char *what) {
     if (d && d->capturing.load())
         return fail(EB_OTHER, "%s: not allowed while the device's stream is being captured", what);
@@ -199,8 +215,8 @@ static void device_destroy(eb_device *d) {
     (void)hipStreamSynchronize(d->stream);
     for (auto &kv : d->pool)
         for (void *p : kv.second) (void)hipFree(p);
-    if (d->ws) (void)hipFree(d->ws);
-    for (float *p : d->ws_retired) (void)hipFree(p);
+    WorkspaceMem mem{d};
+    d->ws.free_all(mem);
     (void)hipStreamDestroy(d->stream);
     delete d;
 }
@@ -534,9 +550,8 @@ static void return_buffers(eb_device *d, std::vector<Parked> &v) {
 // kernels (null when it used none).
 static float *ws_capture_ref(eb_device *d) {
     std::lock_guard<std::mutex> lk(d->ws_mu);
-    float *p = d->ws_in_capture ? d->ws : nullptr;
+    float *p = d->ws_in_capture ? d->ws.ref() : nullptr;
     d->ws_in_capture = false;
-    if (p) ++d->ws_graph_refs[p];
     return p;
 }
 
@@ -545,14 +560,8 @@ static float *ws_capture_ref(eb_device *d) {
 static void ws_graph_unref(eb_device *d, float *p) {
     if (!p) return;
     std::lock_guard<std::mutex> lk(d->ws_mu);
-    auto it = d->ws_graph_refs.find(p);
-    if (it == d->ws_graph_refs.end() || --it->second > 0) return;
-    d->ws_graph_refs.erase(it);
-    auto r = std::find(d->ws_retired.begin(), d->ws_retired.end(), p);
-    if (r != d->ws_retired.end()) {
-        d->ws_retired.erase(r);
-        (void)hipFree(p);
-    }
+    WorkspaceMem mem{d};
+    d->ws.unref(mem, p);
 }
 
 eb_status eb_device_begin_capture(eb_device *dev) {
@@ -987,39 +996,29 @@ static eb_status step_rows_checked(const float *knew, const float *vnew, size_t 
     return EB_OK;
 }
 
-// Grows the device's workspace. Stream ordered: the old buffer is freed only after the
-// stream drains, and not at all while a captured graph still has it in its kernels'
-// arguments (it is then retired, and freed with the last such graph). Returns with
-// dev->ws_mu held in lk.
-static eb_status device_workspace(eb_device *dev, size_t floats, float **out, WsLock &lk) {
+// The device's workspace, grown to hold want floats, or at least least where there is no memory
+// for want; *got: how many of want it holds. Returns with dev->ws_mu held in lk.
+static eb_status device_workspace_up_to(eb_device *dev, size_t want, size_t least, float **out,
+                                        size_t *got, WsLock &lk) {
     lk = WsLock(dev->ws_mu);
-    if (floats > dev->ws_floats) {
-        if (dev->capturing.load())
+    if (dev->capturing.load()) {
+        if (least > dev->ws.floats())
             return fail(EB_OTHER,
                         "the device workspace would have to grow during a graph capture "
                         "(run the captured step once outside the capture first)");
-        if (dev->ws) {
-            if (dev->ws_graph_refs.count(dev->ws)) {
-                dev->ws_retired.push_back(dev->ws);
-            } else {
-                EB_HIP_TRY(hipStreamSynchronize(dev->stream));
-                EB_HIP_TRY(hipFree(dev->ws));
-            }
-            dev->ws = nullptr;
-            dev->ws_floats = 0;
-        }
-        EB_HIP_TRY(hipMalloc((void **)&dev->ws, floats * sizeof(float)));
-        dev->ws_floats = floats;
+        dev->ws_in_capture = true;
+    } else {
+        WorkspaceMem mem{dev};
+        EB_TRY(dev->ws.grow(mem, want, least));
     }
-    if (dev->capturing.load()) dev->ws_in_capture = true;
-    *out = dev->ws;
+    *out = dev->ws.ptr();
+    *got = std::min(want, dev->ws.floats());
     return EB_OK;
 }
 
-// Whether the device's workspace already holds that many floats.
-static bool workspace_holds(eb_device *dev, size_t floats) {
-    std::lock_guard<std::mutex> lk(dev->ws_mu);
-    return dev->ws_floats >= floats;
+static eb_status device_workspace(eb_device *dev, size_t floats, float **out, WsLock &lk) {
+    size_t got;
+    return device_workspace_up_to(dev, floats, floats, out, &got, lk);
 }
 
 // Shared by eb_attn_decode / eb_attn_decode_step: device workspace, then one launch.
@@ -1113,21 +1112,12 @@ static eb_status device_linear(eb_device *dev, const eb_tensor *a,
     EB_TRY(linear_operands_checked(x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f));
     // Room for the split rows, or for the row exponents alone where the launch does not split
     // them or the workspace cannot grow that far (during a capture, or without the memory).
-    size_t wsn = eb::linear_usable_workspace_floats(x, wp, out_f, nseg, m, in_f);
+    const size_t want = eb::linear_usable_workspace_floats(x, wp, out_f, nseg, m, in_f);
+    size_t wsn = 0;
     float *ws = nullptr;
     WsLock lk;
-    if (wsn > 0) {
-        const size_t least = eb::linear_workspace_floats(m, in_f);
-        if (dev->capturing.load() && !workspace_holds(dev, wsn)) wsn = least;
-        eb_status st = device_workspace(dev, wsn, &ws, lk);
-        if (st == EB_OUT_OF_MEMORY && wsn > least) {
-            (void)hipGetLastError();  // (reported by no later call)
-            lk.unlock();
-            wsn = least;
-            st = device_workspace(dev, wsn, &ws, lk);
-        }
-        if (st != EB_OK) return st;
-    }
+    if (want > 0)
+        EB_TRY(device_workspace_up_to(dev, want, eb::linear_workspace_floats(m, in_f), &ws, &wsn, lk));
     return linear_checked(dev->stream, x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f, ws, wsn);
 }
 
