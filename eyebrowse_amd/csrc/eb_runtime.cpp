@@ -135,8 +135,8 @@ using eb::fail;
 // (MAX_POOLED_BYTES, crates/eyebrowse-gpu/src/device.rs:12-14).
 static constexpr size_t kMaxPooledBytes = (size_t)64 << 20;
 
-// A device buffer handed back while a graph capture was running: it stays out of the
-// pool for as long as the graph that may write it exists.
+// A device buffer and, where it was handed back while a graph capture was running (parked): it
+// stays out of the pool for as long as the graph that may write it exists.
 struct Parked {
     void *p;
     size_t bytes;
@@ -155,6 +155,9 @@ struct eb_device {
     // were captured with a buffer of it in their arguments keep that buffer alive. ws_mu.
     eb::Workspace ws;
     bool ws_in_capture = false;  // the running capture handed out the current workspace
+    // Room for split rows that the running capture took where the workspace has none (null:
+    // none so far); its graph holds it afterwards. ws_mu.
+    Parked capture_ws{nullptr, 0, false};
     std::atomic<bool> capturing{false};  // the stream is being captured into a graph
     std::vector<Parked> parked;          // buffers released during the capture (pool_mu)
     std::atomic<eb_recorder *> deferred{nullptr};  // the deferred recorder owning the capture
@@ -217,6 +220,7 @@ static void device_destroy(eb_device *d) {
         for (void *p : kv.second) (void)hipFree(p);
     WorkspaceMem mem{d};
     d->ws.free_all(mem);
+    if (d->capture_ws.p) (void)hipFree(d->capture_ws.p);
     (void)hipStreamDestroy(d->stream);
     delete d;
 }
@@ -319,6 +323,25 @@ size_t eb_device_pooled(eb_device *dev, size_t bytes) {
 
 // ---- tensor ---------------------------------------------------------------------------
 
+static eb_status buffer_alloc(eb_device *dev, size_t bytes, bool from_pool, Parked *out) {
+    void *p = nullptr;
+    const bool poolable = bytes <= kMaxPooledBytes;
+    if (from_pool && poolable) {
+        std::lock_guard<std::mutex> lk(dev->pool_mu);
+        auto it = dev->pool.find(bytes);
+        if (it != dev->pool.end() && !it->second.empty()) {
+            p = it->second.back();
+            it->second.pop_back();
+        }
+    }
+    if (!p) {
+        EB_HIP_TRY(hipSetDevice(dev->ordinal));
+        EB_HIP_TRY(hipMalloc(&p, bytes));
+    }
+    *out = Parked{p, bytes, poolable};
+    return EB_OK;
+}
+
 static eb_status tensor_alloc(eb_device *dev, const size_t *shape, size_t ndim, eb_dtype dt,
                               bool from_pool, eb_tensor **out) {
     if (!dev) return fail(EB_OTHER, "device is null");
@@ -335,28 +358,16 @@ static eb_status tensor_alloc(eb_device *dev, const size_t *shape, size_t ndim, 
     // (crates/eyebrowse-gpu/src/tensor.rs:67).
     size_t bytes = numel * esz;
     if (bytes < esz) bytes = esz;
-    void *p = nullptr;
-    bool poolable = bytes <= kMaxPooledBytes;
-    if (from_pool && poolable) {
-        std::lock_guard<std::mutex> lk(dev->pool_mu);
-        auto it = dev->pool.find(bytes);
-        if (it != dev->pool.end() && !it->second.empty()) {
-            p = it->second.back();
-            it->second.pop_back();
-        }
-    }
-    if (!p) {
-        EB_HIP_TRY(hipSetDevice(dev->ordinal));
-        EB_HIP_TRY(hipMalloc(&p, bytes));
-    }
+    Parked b{nullptr, 0, false};
+    EB_TRY(buffer_alloc(dev, bytes, from_pool, &b));
     auto *t = new eb_tensor();
     t->dev = dev;
     device_retain(dev);
-    t->ptr = p;
+    t->ptr = b.p;
     t->shape.assign(shape, shape + ndim);
     t->dtype = dt;
-    t->bytes = bytes;
-    t->poolable = poolable;
+    t->bytes = b.bytes;
+    t->poolable = b.poolable;
     *out = t;
     return eb::ok();
 }
@@ -581,7 +592,10 @@ eb_status eb_device_end_capture(eb_device *dev, eb_graph **inout) {
     hipError_t e = hipStreamEndCapture(dev->stream, &g);
     std::vector<Parked> held;
     {
+        std::lock_guard<std::mutex> ws_lk(dev->ws_mu);
         std::lock_guard<std::mutex> lk(dev->pool_mu);
+        if (dev->capture_ws.p) dev->parked.push_back(dev->capture_ws);
+        dev->capture_ws = Parked{nullptr, 0, false};
         held.swap(dev->parked);
     }
     dev->capturing.store(false);
@@ -1021,6 +1035,32 @@ static eb_status device_workspace(eb_device *dev, size_t floats, float **out, Ws
     return device_workspace_up_to(dev, floats, floats, out, &got, lk);
 }
 
+// Room for floats that is the running capture's own: its graph keeps it, so that the capture
+// records what the same call does outside one, whatever the workspace holds by then. One buffer
+// serves a capture's calls, which follow each other on the stream. Pooled sizes are powers of
+// two, so that captures of many lengths leave few of them behind. Null without memory. The
+// caller holds dev->ws_mu.
+static float *capture_workspace(eb_device *dev, size_t floats) {
+    Parked &c = dev->capture_ws;
+    size_t bytes = floats * sizeof(float);
+    if (c.bytes < bytes) {
+        if (bytes <= kMaxPooledBytes) {
+            size_t p2 = 4096;
+            while (p2 < bytes) p2 *= 2;
+            bytes = p2;
+        }
+        Parked b{nullptr, 0, false};
+        if (buffer_alloc(dev, bytes, true, &b) != EB_OK) {
+            (void)hipGetLastError();  // (reported by no later call)
+            return nullptr;
+        }
+        std::lock_guard<std::mutex> lk(dev->pool_mu);
+        if (c.p) dev->parked.push_back(c);
+        c = b;
+    }
+    return static_cast<float *>(c.p);
+}
+
 // Shared by eb_attn_decode / eb_attn_decode_step: device workspace, then one launch.
 static eb_status device_decode(eb_device *dev, const float *q, const void *kc, const void *vc,
                                void *kc_w, void *vc_w, const float *knew, const float *vnew,
@@ -1111,13 +1151,19 @@ static eb_status device_linear(eb_device *dev, const eb_tensor *a,
     // (before the workspace grows: by up to m * in_f floats of a call that may be refused)
     EB_TRY(linear_operands_checked(x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f));
     // Room for the split rows, or for the row exponents alone where the launch does not split
-    // them or the workspace cannot grow that far (during a capture, or without the memory).
+    // them or there is no memory. A capture, during which the workspace cannot grow, takes room
+    // of its own.
     const size_t want = eb::linear_usable_workspace_floats(x, wp, out_f, nseg, m, in_f);
     size_t wsn = 0;
     float *ws = nullptr;
     WsLock lk;
-    if (want > 0)
+    if (want > 0) {
         EB_TRY(device_workspace_up_to(dev, want, eb::linear_workspace_floats(m, in_f), &ws, &wsn, lk));
+        if (wsn < want && dev->capturing.load()) {
+            float *own = capture_workspace(dev, want);
+            if (own) ws = own, wsn = want;
+        }
+    }
     return linear_checked(dev->stream, x, xn, wp, wh, yp, yn, out_f, nseg, m, in_f, ws, wsn);
 }
 

@@ -133,7 +133,9 @@ eb_status eb_recorder_new_deferred(eb_device *dev, eb_recorder **out);
  * the device until eb_device_end_capture becomes part of the graph instead of running.
  * While capturing: no host copies (eb_tensor_from_*, to_f32, read_bytes, eb_tensor_write)
  * and no synchronize; a device workspace that would have to grow fails the call (run the
- * step once eagerly first, which also fills the buffer pool). Buffers released during the
+ * step once eagerly first, which also fills the buffer pool; the split rows of projections
+ * are an exception: a capture that finds no room for them takes a buffer of its own, and
+ * records what the eager call does). Buffers released during the
  * capture stay reserved until the graph is released or updated, and so does the device
  * workspace buffer the captured kernels use, also when later work grows the device's
  * workspace (the outgrown buffer is freed with the last graph using it). Kernels take their

@@ -90,8 +90,8 @@ def test_extreme_rows(dev):
 
 
 def test_capture_without_room_for_the_split_rows():
-    """A capture that can use the workspace as it is, but not grow it, still records the product
-    (with the exponents alone); replays give its result."""
+    """A capture that can use the workspace as it is, but not grow it, still records the product;
+    replays give its result."""
     note("linear tiles capture without room")
     dev = eb.Device.new(0)
     m, in_f, out_f = 12, 256, 80
@@ -117,6 +117,72 @@ def test_capture_without_room_for_the_split_rows():
         dev.synchronize()
         assert_close(ct.to_f32().reshape(m, out_f), want, what="replay")
     g.release()
+
+
+def _cold_device():
+    """A device whose workspace holds 2048 floats: row exponents, but no split rows."""
+    dev = eb.Device.new(0)
+    rec = eb.Recorder(dev)
+    eb.linear_f16w(rec, upload(dev, oracle.randn((2048, 8), 1)),
+                   eb.Tensor.from_f16_packed(dev, (8, 8), oracle.randn((8, 8), 2)),
+                   eb.Tensor.empty(dev, (2048, 8)), 2048, 8, 8)
+    rec.submit()
+    return dev
+
+
+def test_a_capture_records_what_an_eager_call_does(dev):
+    """A captured product is the same bits as an eager one, whatever the workspace held when it was
+    captured: several products in one capture, replays between eager work, a recapture."""
+    note("linear tiles capture bits")
+    cold = _cold_device()
+    shapes = [(300, 1024, 100), (12, 256, 80), (700, 2048, 1000)]  # the second within the first's room
+    data = [(oracle.randn((m, k), 3 + i), oracle.randn((n, k), 13 + i) * np.float32(k ** -0.5))
+            for i, (m, k, n) in enumerate(shapes)]
+    want = [_run(dev, x, [w], *x.shape)[0] for x, w in data]
+    xts = [upload(cold, x) for x, _ in data]
+    wts = [eb.Tensor.from_f16_packed(cold, w.shape, w) for _, w in data]
+    cts = [eb.Tensor.empty(cold, (m, n)) for m, _, n in shapes]
+
+    def capture(graph=None):
+        cold.begin_capture()
+        try:
+            rec = eb.Recorder(cold)
+            for xt, wt, ct, (m, k, n) in zip(xts, wts, cts, shapes):
+                eb.linear_f16w(rec, xt, wt, ct, m, k, n)
+            rec.submit()
+        finally:
+            g = cold.end_capture(graph) if graph else cold.end_capture()
+        return g
+
+    graph = capture()
+    other = (oracle.randn((900, 1024), 31), oracle.randn((64, 1024), 32) * np.float32(0.03))
+    for rep in range(4):
+        if rep == 3:
+            graph = capture(graph)
+        for ct, (m, _, n) in zip(cts, shapes):
+            ct.write(np.full((m, n), np.nan, np.float32))
+        graph.launch()
+        for ct, w in zip(cts, want):
+            assert_bitwise(ct.to_f32(), w, f"replay {rep}")
+        # eager work between the replays, which grows the workspace and takes pooled buffers
+        got = _run(cold, other[0], [other[1]], 900, 1024)[0]
+        assert_bitwise(got, _run(dev, other[0], [other[1]], 900, 1024)[0], "eager")
+    graph.release()
+
+
+def test_a_deferred_recorder_does_what_an_eager_call_does(dev):
+    note("linear tiles deferred bits")
+    m, in_f, out_f = 12, 256, 80
+    x, w = oracle.randn((m, in_f), 5), oracle.randn((out_f, in_f), 6) * np.float32(0.03)
+    want = _run(dev, x, [w], m, in_f)[0]
+    cold = _cold_device()
+    xt, wt, ct = upload(cold, x), eb.Tensor.from_f16_packed(cold, w.shape, w), eb.Tensor.empty(cold, (m, out_f))
+    for _ in range(2):
+        ct.write(np.full((m, out_f), np.nan, np.float32))
+        rec = eb.Recorder(cold, deferred=True)
+        eb.linear_f16w(rec, xt, wt, ct, m, in_f, out_f)
+        rec.submit()
+        assert_bitwise(ct.to_f32(), want, "deferred")
 
 
 def test_raw_launch_with_room_for_the_split_rows(dev):
