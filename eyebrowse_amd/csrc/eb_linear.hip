@@ -676,7 +676,10 @@ __device__ __forceinline__ void wait_copies() {
 // (relative error against 64 bits 2.9e-7 in one chain, 2.1e-7 in two at K 1024, 5.8e-7 and
 // 4.1e-7 at 4096). linear_gemm_kernel cuts the contraction at the sizes that these shapes take;
 // the larger shapes keep one chain, as its wide tiles do. A result's bits depend on KW, HALVES,
-// BK and K only, not on the tile.
+// BK and K, not otherwise on the tile. With the eight-wave shapes (kTileFewRows) they are the same
+// whatever the launch's other outputs; beyond, the tile (so HALVES) is chosen for all outputs
+// together, and a fused and a separate projection of many rows may differ in their last bits
+// (linear_gemm_kernel's wide tiles and cut contraction do so too).
 // Workgroups: each XCD gets a contiguous range of tiles, in groups of kGroupM row tiles by all
 // feature tiles, row tile fastest, so that the tiles in flight on an XCD share rows and features.
 constexpr int kGroupM = 4;
@@ -861,16 +864,20 @@ eb_status launch_tile(hipStream_t st, const _Float16 *xs, const float *ex, Linea
 }
 
 // The tile shapes, and the time of one round of tiles (one per CU) as fixed + per_k * K us, fitted
-// to a sweep of 9 to 4096 rows at the Qwen and Mistral widths. tile_cost takes the rounds of the
-// fullest CU, or half way to the average where two workgroups share a CU and overlap.
+// to a sweep of 9 to 4096 rows at the Qwen and Mistral widths (made before the shapes with HALVES
+// cut their sums in two; not fitted again since). tile_cost takes the rounds of the fullest CU, or
+// half way to the average where two workgroups share a CU and overlap.
 struct TileModel {
     int bm, bn;
     bool shared;  // two workgroups per CU
     float fixed, per_k;
 };
 // Up to kTileFewRows rows and whole 128-deep stages: eight waves share each stage's steps, which
-// keeps a CU's copies in flight on the small tiles that few rows need (Qwen o_proj, 256 rows: 11.6
-// us, against 18.9 with the one-sum shapes). Beyond, one chain of sums per output.
+// keeps a CU's copies in flight on the small tiles that few rows need. Beyond, one wave sums an
+// output. The line is a number of rows, so that it does not move with the launch's other outputs.
+// Both sides of it (us, split pass included, eight waves / one): Mistral o_proj 128 rows 18.8 /
+// 29.9, 256 rows 27.5 / 31.3; q/k/v 24.9 / 29.8, 45.5 / 44.8; Qwen o_proj 10.2 / 17.8, 10.4 /
+// 18.9; 1536 -> 6144, the worst for eight waves, 14.0 / 15.2, 23.6 / 21.5.
 using TileK8a = TileShape<1, 1, 1, 1, 8, 128, 4>;
 using TileK8b = TileShape<1, 1, 1, 2, 8, 128, 4>;
 using TileK8c = TileShape<1, 1, 2, 2, 8, 128, 3>;

@@ -103,10 +103,9 @@ def test_qwen_prompt_projection_sampled_rows(dev):
 
 
 def test_qwen_o_proj_split_contraction(dev):
-    """Qwen3 o_proj at T=4096 (4096 x 2048 -> 1024): one 128 x 128 tile per CU, so the
-    contraction is cut in two halves whose partials add into the zeroed output. Sampled
-    rows against the oracle, and a second launch bit-identical (two addends onto zero give
-    the same bits in either order)."""
+    """Qwen3 o_proj at T=4096 (4096 x 2048 -> 1024) on the split rows: sampled rows against the
+    oracle, and a second launch bit-identical. (The contraction cut over two workgroups, which
+    launches without room for split rows use, is test_unsplit_rows_match_oracle's.)"""
     note("linear gemm qwen o_proj T=4096 (split contraction)")
     m, in_f, out_f = 4096, 2048, 1024
     x = oracle.randn((m, in_f), 7)
@@ -254,8 +253,9 @@ def test_empty_and_invalid(dev):
     (2000, (4096, 2000, 4000)),  # ragged rows and features on the wide tiles
 ])
 def test_wide_tile_gemm_sampled_rows(dev, m, outs):
-    """Grids with at least two wide tiles per CU take the 64 x 128-per-wave kernel; rows
-    sampled across the tiles (first, last, tile edges) against the oracle."""
+    """Fused projections of many rows on the split rows' widest tiles; rows sampled across the
+    tiles (first, last, tile edges) against the oracle. (The wide tiles of launches without room
+    for split rows are test_unsplit_rows_match_oracle's.)"""
     note(f"linear wide gemm m={m} outs={outs}")
     in_f = 1024
     x = oracle.randn((m, in_f), 60)
@@ -285,3 +285,40 @@ def test_few_rows_bits_do_not_depend_on_the_call(dev, in_f, out_f):
     for m in (1, 2, 3, 4, 5, 8):
         got = run(dev, x[:m], w, m, in_f, out_f)
         assert_bitwise(got[:, :1001], want[:m], f"{m} rows")
+
+
+def run_raw(dev, x, w, m, in_f, out_f):
+    """A raw launch with room for the row exponents alone; the output starts as NaN."""
+    xt, wt = upload(dev, x), eb.Tensor.from_f16_packed(dev, w.shape, w)
+    ct = upload(dev, np.full((m, out_f), np.nan, np.float32))
+    need = eb.linear_workspace_floats(m, in_f)
+    ws = upload(dev, np.full(need, np.nan, np.float32))
+    eb.launch_linear_f16w(dev.stream, xt.data_ptr, xt.numel(), wt.data_ptr, 2 * wt.numel(),
+                          ct.data_ptr, ct.numel(), m, in_f, out_f, ws.data_ptr, need)
+    dev.synchronize()
+    return ct.to_f32().reshape(m, out_f)
+
+
+@pytest.mark.parametrize("m,in_f,out_f", [
+    (4096, 1024, 4096),   # two wide tiles (128 x 256) per CU
+    (2000, 1024, 8200),   # wide, ragged rows and features
+    (4096, 1032, 4096),   # wide, a contraction that is not whole stages
+    (4096, 2048, 1024),   # one 128 x 128 tile per CU: the contraction cut in two halves
+    (4000, 2056, 1016),   # cut, ragged rows, features and contraction
+    (1000, 4096, 700),    # cut, 48 tiles
+])
+def test_unsplit_rows_match_oracle(dev, m, in_f, out_f):
+    """Without room for split rows (a raw launch with the exponents alone, and every launch whose
+    contraction is no multiple of 64) the kernel splits the rows it stages: its wide tiles, and its
+    cut contraction, whose halves add into the zeroed output. Sampled rows against the oracle, and
+    a second launch bit-identical (two addends onto zero give the same bits in either order)."""
+    note(f"linear unsplit rows m={m} in={in_f} out={out_f}")
+    x = oracle.randn((m, in_f), 71)
+    w = oracle.randn((out_f, in_f), 72) * np.float32(in_f ** -0.5)
+    got = run_raw(dev, x, w, m, in_f, out_f)
+    assert np.isfinite(got).all()
+    assert_bitwise(run_raw(dev, x, w, m, in_f, out_f), got, "second launch")
+    if in_f % 64:
+        assert_bitwise(run(dev, x, w, m, in_f, out_f), got, "recorder")
+    rows = sorted({0, 1, 127, 128, 129, m // 2, m - 129, m - 2, m - 1})
+    assert_close(got[rows], want_of(x[rows], w, len(rows), in_f, out_f), what="unsplit rows")

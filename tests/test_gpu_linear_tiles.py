@@ -1,6 +1,6 @@
 """linear_f16w on split rows copied memory-to-LDS (linear_tile_kernel): every tile shape at its
-edges against the oracle, the same bits whatever the launch's other outputs, and the path
-without room for the split rows."""
+edges against the oracle, the same bits beside other outputs where the tiles sum alike, and calls
+that find no room for the split rows."""
 import numpy as np
 import pytest
 
@@ -59,8 +59,10 @@ def test_tiles_match_oracle(dev, m, in_f, outs):
 
 @pytest.mark.parametrize("m", [40, 256, 257, 700])
 def test_bits_do_not_depend_on_the_launch(dev, m):
-    """An output's sums are the same whether it is launched alone or beside others (other tile
-    shapes)."""
+    """An output's sums are the same whether it is launched alone or beside others, where the tiles
+    of both launches sum alike: all of those for up to 256 rows, and the smaller three beyond (other
+    widths of row and feature; the two largest sum in one chain, so a fused and a separate
+    projection may differ in their last bits on long prompts)."""
     note(f"linear tiles alone and together m={m}")
     in_f, outs = 1024, (2048, 100, 3000)
     x = oracle.randn((m, in_f), 5)
