@@ -37,6 +37,9 @@ def _chunk(dev, q, kc, vc, dtype, h, hkv, pos0, rows, hd, max_seq, scale, window
     (2, 2, 80, 7, 300, 0),      # GQA 1, padded head dim, records
     (4, 2, 256, 3, 64, 0),      # one block at 256: staged
     (4, 2, 256, 95, 97, 0),     # two blocks at 256: records
+    (128, 8, 128, 10, 545, 0),  # more than 512 blocks of 4 heads: records without a key split
+    (128, 8, 128, 70, 530, 90),  # the same, windowed
+    (64, 16, 64, 0, 1030, 0),   # the same at 64, from position 0
 ])
 def test_same_bits_as_f32_cache(dev, dtype, h, hkv, hd, pos0, rows, window):
     note(f"half images {dtype.name} hd={hd} pos0={pos0} rows={rows} window={window}")
