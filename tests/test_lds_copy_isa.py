@@ -55,7 +55,7 @@ def test_the_check_sees_both_hazards():
 def kernels(tmp_path_factory):
     """name -> [(mnemonic, operands)] of every kernel with such copies."""
     d = tmp_path_factory.mktemp("isa")
-    eb.lib()  # (builds it if nothing is built)
+    eb.lib()  # (says how to build it if it is missing)
     src = os.path.join(os.path.dirname(os.path.abspath(eb.__file__)), "libeyebrowse_hip.so")
     os.symlink(src, d / "lib.so")
     subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=d, check=True, capture_output=True)
